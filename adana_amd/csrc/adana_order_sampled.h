@@ -1,0 +1,1173 @@
+// adana_order_sampled.h -- order statistics in two reads of the tensors.
+// Included by adana_order_stats.hip (kernels and host code of
+// adana_order_stats_sampled; order_key, key_to_bits, check and the radix
+// select it falls back on are that file's).
+//
+// The radix select reads every tensor 5 to 6 times, because equal-width digits
+// of the key do not fit the values: a tau tensor's values crowd into a few
+// exponents, so the early digits separate nothing.  Here a sample of the
+// tensor first fits the bins to the values:
+//
+//   1. sample_map_kernel, one workgroup per tensor: 4,096 sampled keys give
+//      the tensor's map from key to bin: 1,024 equal cells over the sample's
+//      range, each cell divided into as many equal bins as its share of the
+//      sample earns (up to 8,192 bins in all).  The map is monotone in the
+//      key, whatever the sample, so it decides speed and never results.  A
+//      tensor of at most kSortMax values is sorted in LDS instead and done.
+//   2. sampled_hist_kernel, first read: exact counts per bin.
+//   3. sampled_walk_kernel, one workgroup per tensor: every wanted rank's bin
+//      and its rank inside it.  The wanted bins (a few per cent of the values)
+//      become segments of the candidate buffer.
+//   4. sampled_collect_kernel, second read: the values of the wanted bins,
+//      into their segments.
+//   5. segment_few_kernel and segment_many_kernel, one workgroup per segment:
+//      the ranks' values.
+//
+// Nothing comes back to the host between the launches.  A key that repeats
+// through the sample (zeros of rows that never had a gradient) is counted
+// beside the bins instead of collected.  A tensor whose values do not fit this
+// (many repeated values; wanted bins over 1/8 of its values; a segment too
+// crowded to finish in LDS) is marked, and the host runs the radix select on
+// the marked ones.
+//
+// Measured: the 1.31G tau values of a 1.3B-parameter model's 146 tensors take
+// 2.8 ms (7.4 ms with the radix select's 6 passes): the first read 0.83 ms (6.3
+// TB/s, memory-bound), the second 1.27 ms (its loop alone 0.81; the rest is the
+// candidates' scattered writes), the selects 0.2 ms, the copies, launches and
+// host work about 0.4 ms.  One tensor of 4M values: 0.13 ms (radix 0.45), seven
+// launches of 7 to 16 us and two copies.
+
+namespace sampled {
+
+constexpr int kMapThreads = 1024;
+constexpr int kSample = 4096;                // sampled keys per tensor (16,384: the map takes 45 us longer, all else 40 us less)
+constexpr int kPer = kSample / kMapThreads;
+constexpr int kTrim = 2;                     // samples left outside the cells at either end
+constexpr int kSortMax = 8192;               // tensors up to this size are sorted in LDS
+constexpr int kCells = 1024;
+constexpr int kMaxBins = 8192;
+constexpr int kSubBits = 12;                 // a cell is divided on its top 12 bits
+constexpr int kMaxRanks = 1024;              // per tensor (one thread per rank)
+constexpr int kHeavy = 2;                    // repeated keys counted beside the bins
+constexpr uint32_t kHeavyMin = 16;           // of the sample: such a key is repeated
+constexpr int kHistThreads = 512;
+constexpr int kHistIter = kHistThreads * 16;     // values per iteration of the first read
+constexpr int kCollectThreads = 512;
+constexpr int kStage = 4608;                 // second read: candidates staged in LDS per workgroup
+constexpr int kFlushEvery = 10;              // and how many iterations apart they are looked at
+constexpr int kSegThreads = 1024;
+constexpr int kSmallThreads = 256;           // segments of few ranks and candidates: these many threads,
+constexpr int kSmallPer = 16;                // each holding up to so many candidates
+constexpr uint32_t kSegMax = 1u << 18;       // a larger segment is left to the radix select: one workgroup reads it
+constexpr int64_t kMaxElems = int64_t{1} << 28;  // larger tensors' segments would be; they take the radix select at once
+constexpr int64_t kFewGrid = 2048, kManyGrid = 512;
+constexpr int kSegSort = 4096;               // candidates of a large segment sorted in LDS at a time
+constexpr int kSegDigit = 11;                // digit of a segment's own radix select
+constexpr int kPartBits = 13;                // parts of a segment of many ranks
+constexpr int64_t kCandDen = 8;              // candidate buffer: 1 / kCandDen of a tensor's values
+
+enum State : uint32_t { kRun = 0, kDone = 1, kRadix = 2 };   // kRadix: left to the radix select
+
+// One tensor: what the host gives, and the map (sample_map_kernel).
+struct Tensor {
+    const float *x;
+    uint64_t n;
+    uint64_t cand_first;          // its candidate buffer's first entry, and size
+    uint64_t cand_cap;
+    int32_t rank_first, n_ranks;
+    uint32_t bin_budget;          // bins the map may use
+    uint32_t bin_first;           // its first entry of hist and wanted
+    uint32_t map;                 // its row of cell
+    uint32_t key0, shift, bins;   // cell = (key - key0) >> shift, clamped
+    uint32_t n_heavy;
+    uint32_t heavy_key[kHeavy];
+    uint32_t heavy_count[kHeavy];
+};
+
+// One tile of the reads: elements [first, last) of a tensor.
+struct Tile {
+    int32_t tensor;
+    int32_t pad;
+    uint64_t first, last;
+};
+
+// The candidates of one wanted bin, and the ranks they hold.
+struct Segment {
+    uint64_t first;               // in the candidate buffer
+    uint32_t count;
+    uint32_t rank_first, n_ranks; // ranks in order
+    uint32_t tensor;
+    uint32_t n_heavy;             // repeated keys of this bin (not among the candidates)
+    uint32_t heavy_key[kHeavy];
+    uint32_t heavy_count[kHeavy];
+};
+
+struct Args {
+    Tensor *tensor;
+    const Tile *tile;
+    const uint32_t *rank;         // ascending per tensor
+    uint32_t *residual;           // per rank: its rank within its segment
+    uint2 *cell;                  // [map][kCells] {bins of the cell, first bin << kSubBits}
+    uint32_t *hist;               // [bin_first + bin]
+    uint16_t *wanted;             // [bin_first + bin]: 1 + segment of the bin within the tensor, 0: not wanted
+    Segment *seg;                 // one slot per rank
+    uint32_t *cursor;             // per segment slot: candidates placed
+    uint32_t *few, *many;         // slots of the segments for either select kernel
+    uint32_t *n_few;              // their numbers: [0] few, [1] many
+    uint32_t *cand;               // candidate keys
+    uint32_t *out;                // per rank: the value's bits
+    uint32_t *state;              // per tensor: State
+    int32_t n;
+};
+
+__device__ __forceinline__ uint32_t key_bits(uint32_t key) {
+    return (key & 0x80000000u) ? (key & 0x7fffffffu) : ~key;
+}
+
+__device__ __forceinline__ uint32_t mix32(uint32_t x) {
+    x ^= x >> 16;
+    x *= 0x85ebca6bu;
+    x ^= x >> 13;
+    x *= 0xc2b2ae35u;
+    return x ^ (x >> 16);
+}
+
+// The map, monotone in key: keys below key0 and past the last cell clamp to
+// the two outer cells, which have one bin each.  For values in [0, +inf] the
+// key is the bits with the sign set, so there bin_of_bits takes the bits
+// themselves against key0 without its sign (key0 has it whenever the sample
+// has no negative values).
+struct Map {
+    uint32_t key0, shift;
+    __device__ __forceinline__ uint32_t at(uint32_t d, const uint2 *cell) const {
+        const uint2 e = cell[min(d >> shift, static_cast<uint32_t>(kCells - 1))];
+        const uint32_t sub = (d >> (shift - kSubBits)) & ((1u << kSubBits) - 1);
+        return (__umul24(sub, e.x) + e.y) >> kSubBits;        // 12 x 13 bits: no overflow
+    }
+    __device__ __forceinline__ uint32_t bin(uint32_t key, const uint2 *cell) const {
+        return at(__builtin_elementwise_sub_sat(key, key0), cell);
+    }
+    __device__ __forceinline__ bool takes_bits() const { return key0 >= 0x80000000u; }
+    __device__ __forceinline__ uint32_t bin_of_bits(uint32_t bits, const uint2 *cell) const {
+        return at(__builtin_elementwise_sub_sat(bits, key0 & 0x7fffffffu), cell);
+    }
+};
+
+__device__ __forceinline__ uint32_t wave_min(uint32_t v) {
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) v = min(v, static_cast<uint32_t>(__shfl_xor(v, o, 64)));
+    return v;
+}
+__device__ __forceinline__ uint32_t wave_max(uint32_t v) {
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) v = max(v, static_cast<uint32_t>(__shfl_xor(v, o, 64)));
+    return v;
+}
+
+// Sum of v over the workgroup's threads before this one; total in *all.
+template <int NT>
+__device__ __forceinline__ uint32_t block_scan(uint32_t v, uint32_t *waves, uint32_t *all) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    uint32_t incl = v;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const uint32_t u = __shfl_up(incl, o, 64);
+        if (lane >= o) incl += u;
+    }
+    __syncthreads();                                 // waves[] may still be read from an earlier call
+    if (lane == 63) waves[wave] = incl;
+    __syncthreads();
+    uint32_t before = 0, sum = 0;
+#pragma unroll
+    for (int w = 0; w < NT / 64; ++w) {
+        before += w < wave ? waves[w] : 0u;
+        sum += waves[w];
+    }
+    *all = sum;
+    return before + incl - v;
+}
+
+// Ascending bitonic sort of p (a power of two) keys in LDS.  Steps over
+// distances up to 64 keep each wave inside its own 128 keys, so only the
+// longer ones need the workgroup's barrier.
+template <int NT>
+__device__ __forceinline__ void lds_sort(uint32_t *x, int p) {
+    for (int k = 2; k <= p; k <<= 1) {
+        for (int j = k >> 1; j > 0; j >>= 1) {
+            if (j >= 64 || j == k >> 1) __syncthreads();
+            else __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            for (int i = threadIdx.x; i < p / 2; i += NT) {
+                const int a = ((i & ~(j - 1)) << 1) | (i & (j - 1)), b = a | j;
+                const uint32_t u = x[a], v = x[b];
+                const bool up = (a & k) == 0;
+                if (up ? u > v : u < v) {
+                    x[a] = v;
+                    x[b] = u;
+                }
+            }
+        }
+    }
+    __syncthreads();
+}
+
+__device__ __forceinline__ int pow2_at_least(uint32_t n) {
+    return n <= 2 ? 2 : 1 << (32 - __builtin_clz(n - 1));
+}
+
+__global__ __launch_bounds__(kMapThreads) void sample_map_kernel(Args a) {
+    __shared__ uint32_t x[kSortMax];                 // small tensor: its keys; else cell counts and picks
+    __shared__ uint32_t waves[kMapThreads / 64];
+    __shared__ uint32_t s_lo, s_hi, s_heavy, s_hk[kHeavy];
+    const int t = blockIdx.x, tid = threadIdx.x;
+    Tensor &T = a.tensor[t];
+    const float *v = T.x;
+    const uint32_t n = static_cast<uint32_t>(T.n);
+    if (n <= static_cast<uint32_t>(kSortMax)) {
+        const int p = pow2_at_least(n);
+        for (int i = tid; i < p; i += kMapThreads) x[i] = i < static_cast<int>(n) ? order_key(v[i]) : 0xffffffffu;
+        lds_sort<kMapThreads>(x, p);
+        for (int j = tid; j < T.n_ranks; j += kMapThreads) {
+            const int r = T.rank_first + j;
+            a.out[r] = key_bits(x[a.rank[r]]);
+        }
+        if (tid == 0) a.state[t] = kDone;
+        return;
+    }
+    // one key at a scattered place of each of kSample equal stretches
+    uint32_t key[kPer];
+    const uint32_t step = n / kSample;
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) {
+        const uint32_t at = tid + i * kMapThreads;
+        key[i] = order_key(v[static_cast<uint64_t>(at) * n / kSample + mix32(at) % step]);
+    }
+    // the sample's range, kTrim keys left out at either end, first to the
+    // nearest 2^20 keys and then to the keys inside
+    for (int i = tid; i < 4096; i += kMapThreads) x[i] = 0;
+    if (tid == 0) {
+        s_lo = 0xffffffffu;
+        s_hi = 0;
+        s_heavy = 0;
+    }
+    __syncthreads();
+    // a clustered tensor's keys share a handful of these: one add per wave for
+    // the first few (64 adds to one LDS address cost 64 times one)
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) {
+        const uint32_t d = key[i] >> 20;
+        bool left = true;
+        for (int round = 0; round < 4; ++round) {
+            const uint64_t todo = __ballot(left);
+            if (todo == 0) break;
+            const uint32_t pick = __shfl(d, __ffsll(static_cast<unsigned long long>(todo)) - 1, 64);
+            const uint64_t same = __ballot(left && d == pick);
+            if (left && d == pick) {
+                if ((tid & 63) == __ffsll(static_cast<unsigned long long>(same)) - 1)
+                    atomicAdd(&x[d], static_cast<uint32_t>(__popcll(same)));
+                left = false;
+            }
+        }
+        if (left) atomicAdd(&x[d], 1u);
+    }
+    __syncthreads();
+    uint32_t all;
+    uint32_t q[4], sum = 0;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) sum += q[k] = x[4 * tid + k];
+    uint32_t before = block_scan<kMapThreads>(sum, waves, &all);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        const uint32_t upto = before + q[k];
+        if (before <= kTrim && upto > kTrim) s_lo = static_cast<uint32_t>(4 * tid + k);
+        if (before < kSample - kTrim && upto >= kSample - kTrim) s_hi = static_cast<uint32_t>(4 * tid + k);
+        before = upto;
+    }
+    __syncthreads();
+    const uint32_t lo20 = s_lo, hi20 = s_hi;
+    __syncthreads();
+    if (tid == 0) {
+        s_lo = 0xffffffffu;
+        s_hi = 0;
+    }
+    __syncthreads();
+    uint32_t mn = 0xffffffffu, mx = 0;
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) {
+        if ((key[i] >> 20) >= lo20 && (key[i] >> 20) <= hi20) {
+            mn = min(mn, key[i]);
+            mx = max(mx, key[i]);
+        }
+    }
+    mn = wave_min(mn);
+    mx = wave_max(mx);
+    if ((tid & 63) == 0) {
+        atomicMin(&s_lo, mn);
+        atomicMax(&s_hi, mx);
+    }
+    // x: [0, kCells) counts, [kCells, 2 kCells) a key of the cell, [2 kCells, 3 kCells) its repeats
+    for (int i = tid; i < 3 * kCells; i += kMapThreads) x[i] = 0;
+    __syncthreads();
+    const uint32_t key_lo = s_lo, range = s_hi - key_lo;
+    uint32_t shift = kSubBits;
+    while ((range >> shift) > kCells - 3) ++shift;
+    // one cell below the sample's range, but none below +0 for a sample without
+    // negative values (Map::takes_bits)
+    const uint32_t floor0 = key_lo >= 0x80000000u ? 0x80000000u : 0u;
+    const uint32_t key0 = key_lo - floor0 >= (1u << shift) ? key_lo - (1u << shift) : floor0;
+    uint32_t c[kPer];
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) {
+        c[i] = min(__builtin_elementwise_sub_sat(key[i], key0) >> shift, static_cast<uint32_t>(kCells - 1));
+        atomicAdd(&x[c[i]], 1u);
+        x[kCells + c[i]] = key[i];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < kPer; ++i)
+        if (x[kCells + c[i]] == key[i]) atomicAdd(&x[2 * kCells + c[i]], 1u);
+    __syncthreads();
+    static_assert(kCells == kMapThreads, "one cell per thread");
+    uint32_t count = x[tid];
+    if (x[2 * kCells + tid] >= kHeavyMin) {
+        const uint32_t k = atomicAdd(&s_heavy, 1u);
+        if (k < kHeavy) s_hk[k] = x[kCells + tid];
+        count -= x[2 * kCells + tid];
+    }
+    const uint32_t budget = T.bin_budget - kCells;
+    uint32_t nb = max(1u, count * budget / kSample);
+    nb = min(nb, 1u << kSubBits);
+    if (tid == 0 || tid == kCells - 1) nb = 1;
+    const uint32_t base = block_scan<kMapThreads>(nb, waves, &all);
+    a.cell[static_cast<int64_t>(T.map) * kCells + tid] = make_uint2(nb, base << kSubBits);
+    for (uint32_t i = tid; i < all; i += kMapThreads) a.hist[static_cast<int64_t>(T.bin_first) + i] = 0;
+    if (tid == 0) {
+        T.key0 = key0;
+        T.shift = shift;
+        T.bins = all;
+        T.n_heavy = min(s_heavy, static_cast<uint32_t>(kHeavy));
+        for (int k = 0; k < kHeavy; ++k) {
+            T.heavy_key[k] = s_hk[k];
+            T.heavy_count[k] = 0;
+        }
+        a.state[t] = s_heavy > kHeavy ? kRadix : kRun;
+    }
+}
+
+// Whether 4 values are all in [0, +inf].
+__device__ __forceinline__ bool plain4(const F4 &q) {
+    const uint32_t m = max(max(__float_as_uint(q[0]), __float_as_uint(q[1])),
+                           max(__float_as_uint(q[2]), __float_as_uint(q[3])));
+    return m <= 0x7f800000u;
+}
+
+__device__ __forceinline__ uint32_t key_of(uint32_t bits) { return order_key(__uint_as_float(bits)); }
+
+// Takes f over the values [first, last) of x, VECS 16-byte loads per thread at
+// a time; done(last) follows every kFlushEvery iterations and the last one.
+// All threads of the workgroup take part in every call.  f.vecs<PLAIN>(bits,
+// in): the values' bits, PLAIN if all are in [0, +inf], `in` (per load) where
+// the thread has values; f.single(bits, in): one value.
+template <int NT, int VECS, typename F, typename G>
+__device__ __forceinline__ void for_values(const float *x, uint64_t n, uint64_t first, uint64_t last, bool takes_bits,
+                                           F &f, G done) {
+    // the tensor's aligned part starts `head` values in; tile bounds count from
+    // there, and the first tile takes the head, the last one the tail
+    const uint64_t head = min(static_cast<uint64_t>((4 - ((reinterpret_cast<uintptr_t>(x) >> 2) & 3)) & 3), n);
+    const int tid = threadIdx.x;
+    const float *y = x + head;
+    const uint64_t body = n - head;
+    const uint64_t lo = first, hi = min(last, body);             // [lo, hi) of y, lo a multiple of 4
+    const uint64_t vec_hi = lo + ((hi > lo ? hi - lo : 0) & ~3ull);
+    constexpr uint64_t kIter = static_cast<uint64_t>(VECS) * 4 * NT;
+    int since = 0;
+    for (uint64_t b = lo; b < vec_hi; b += kIter) {
+        const bool whole = b + kIter <= vec_hi;                  // uniform
+        F4 q[VECS];
+        if (whole) {
+#pragma unroll
+            for (int u = 0; u < VECS; ++u)
+                q[u] = __builtin_nontemporal_load(
+                    (const GLOBAL_AS F4 *)(y + b + (static_cast<uint64_t>(u) * NT + tid) * 4));
+        } else {
+#pragma unroll
+            for (int u = 0; u < VECS; ++u) {
+                const uint64_t e = b + (static_cast<uint64_t>(u) * NT + tid) * 4;
+                q[u] = F4{0.0f, 0.0f, 0.0f, 0.0f};
+                if (e < vec_hi) q[u] = __builtin_nontemporal_load((const GLOBAL_AS F4 *)(y + e));
+            }
+        }
+        bool plain = whole && takes_bits;
+#pragma unroll
+        for (int u = 0; u < VECS; ++u) plain = plain && plain4(q[u]);
+        uint32_t bits[VECS * 4];
+#pragma unroll
+        for (int e = 0; e < VECS * 4; ++e) bits[e] = __float_as_uint(q[e >> 2][e & 3]);
+        bool in[VECS];
+        if (__ballot(!plain) == 0) {
+#pragma unroll
+            for (int u = 0; u < VECS; ++u) in[u] = true;
+            f.template vecs<true>(bits, in);
+        } else {
+#pragma unroll
+            for (int u = 0; u < VECS; ++u) in[u] = b + (static_cast<uint64_t>(u) * NT + tid) * 4 < vec_hi;
+            f.template vecs<false>(bits, in);
+        }
+        if (++since == kFlushEvery) {
+            done(false);
+            since = 0;
+        }
+    }
+    // up to three values before the aligned part (first tile) and after it
+    const bool one_head = first == 0 && tid < static_cast<int>(head);
+    const bool one_tail = !one_head && tid >= 64 && vec_hi + (tid - 64) < hi;
+    const uint32_t one = one_head ? __float_as_uint(x[tid]) : one_tail ? __float_as_uint(y[vec_hi + (tid - 64)]) : 0u;
+    f.single(one, one_head || one_tail);
+    done(true);
+}
+
+struct HistOp {
+    uint32_t *h;
+    const uint2 *cell;
+    Map map;
+    uint32_t n_heavy, hk0, hk1;
+    uint32_t hc0, hc1;            // this thread's repeated keys
+    __device__ __forceinline__ void one(uint32_t key) {
+        if (n_heavy) {
+            if (key == hk0) {
+                ++hc0;
+                return;
+            }
+            if (key == hk1) {
+                ++hc1;
+                return;
+            }
+        }
+        atomicAdd(&h[map.bin(key, cell)], 1u);
+    }
+    template <bool PLAIN, int N, int V>
+    __device__ __forceinline__ void vecs(const uint32_t (&bits)[N], const bool (&in)[V]) {
+        if (PLAIN && n_heavy == 0) {
+            uint32_t b[N];
+#pragma unroll
+            for (int e = 0; e < N; ++e) b[e] = map.bin_of_bits(bits[e], cell);
+#pragma unroll
+            for (int e = 0; e < N; ++e)
+                if (in[e >> 2]) atomicAdd(&h[b[e]], 1u);
+        } else {
+#pragma unroll
+            for (int e = 0; e < N; ++e)
+                if (in[e >> 2]) one(key_of(bits[e]));
+        }
+    }
+    __device__ __forceinline__ void single(uint32_t bits, bool in) {
+        if (in) one(key_of(bits));
+    }
+};
+
+__global__ __launch_bounds__(kHistThreads) void sampled_hist_kernel(Args a) {
+    extern __shared__ uint32_t lds[];                // [2 kCells] cells, [bins] counts
+    const Tile tile = a.tile[blockIdx.x];
+    Tensor &T = a.tensor[tile.tensor];
+    if (a.state[tile.tensor] != kRun) return;
+    const int tid = threadIdx.x;
+    uint2 *cell = reinterpret_cast<uint2 *>(lds);
+    uint32_t *h = lds + 2 * kCells;
+    const uint32_t bins = T.bins;
+    for (int i = tid; i < kCells; i += kHistThreads) cell[i] = a.cell[static_cast<int64_t>(T.map) * kCells + i];
+    for (uint32_t i = tid; i < bins; i += kHistThreads) h[i] = 0;
+    __syncthreads();
+    const uint32_t nh = T.n_heavy;
+    const Map map{T.key0, T.shift};
+    HistOp op{h, cell, map, nh, T.heavy_key[0], nh > 1 ? T.heavy_key[1] : T.heavy_key[0], 0, 0};
+    for_values<kHistThreads, 4>(T.x, T.n, tile.first, tile.last, map.takes_bits(), op, [](bool) {});
+    __syncthreads();
+    uint32_t *g = a.hist + static_cast<int64_t>(T.bin_first);
+    for (uint32_t i = tid; i < bins; i += kHistThreads)
+        if (h[i]) atomicAdd(&g[i], h[i]);
+    if (nh) {
+#pragma unroll
+        for (int k = 0; k < kHeavy; ++k) {
+            uint32_t s = k == 0 ? op.hc0 : op.hc1;
+#pragma unroll
+            for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+            if ((tid & 63) == 0 && s) atomicAdd(&T.heavy_count[k], s);
+        }
+    }
+}
+
+// Whether segment_few_kernel takes a segment (segment_many_kernel the others).
+__device__ __forceinline__ bool few(const Segment &s) {
+    return s.n_ranks <= 4 && s.count <= static_cast<uint32_t>(kSmallThreads * kSmallPer);
+}
+
+__global__ __launch_bounds__(kMapThreads) void sampled_walk_kernel(Args a) {
+    constexpr int kBinsPer = kMaxBins / kMapThreads;
+    __shared__ uint32_t below[kMaxBins + 1];         // values before each bin (repeated keys included)
+    __shared__ uint32_t waves[kMapThreads / 64];
+    __shared__ uint32_t rank_bin[kMaxRanks];
+    __shared__ uint32_t seg_rank[kMaxRanks + 1];     // first rank of each segment
+    __shared__ uint32_t hbin[kHeavy];
+    const int t = blockIdx.x, tid = threadIdx.x;
+    const Tensor &T = a.tensor[t];
+    if (a.state[t] == kDone) return;
+    const int nr = T.n_ranks;
+    if (tid < nr) a.cursor[T.rank_first + tid] = 0;
+    if (a.state[t] != kRun) return;                  // uniform
+    const uint32_t bins = T.bins;
+    const uint32_t *h = a.hist + static_cast<int64_t>(T.bin_first);
+    uint16_t *wanted = a.wanted + static_cast<int64_t>(T.bin_first);
+    if (tid < kHeavy)
+        hbin[tid] = tid < static_cast<int>(T.n_heavy)
+                        ? Map{T.key0, T.shift}.bin(T.heavy_key[tid], a.cell + static_cast<int64_t>(T.map) * kCells)
+                        : 0xffffffffu;
+    __syncthreads();
+    uint32_t c[kBinsPer], sum = 0, all;
+#pragma unroll
+    for (int k = 0; k < kBinsPer; ++k) {
+        const uint32_t b = tid * kBinsPer + k;
+        uint32_t v = b < bins ? h[b] : 0u;
+        for (int q = 0; q < kHeavy; ++q)
+            if (b == hbin[q]) v += T.heavy_count[q];
+        c[k] = v;
+        sum += v;
+    }
+    uint32_t before = block_scan<kMapThreads>(sum, waves, &all);
+#pragma unroll
+    for (int k = 0; k < kBinsPer; ++k) {
+        below[tid * kBinsPer + k] = before;
+        before += c[k];
+    }
+    if (tid == 0) below[kMaxBins] = all;
+    for (uint32_t b = tid; b < bins; b += kMapThreads) wanted[b] = 0;
+    __syncthreads();
+    // this thread's rank: the last bin that starts at or before it
+    uint32_t bin = 0xffffffffu;
+    if (tid < nr) {
+        const uint32_t r = a.rank[T.rank_first + tid];
+        uint32_t l = 0, u = bins - 1;
+        while (l < u) {
+            const uint32_t mid = (l + u + 1) >> 1;
+            if (below[mid] <= r) l = mid; else u = mid - 1;
+        }
+        bin = l;
+        rank_bin[tid] = bin;
+        a.residual[T.rank_first + tid] = r - below[bin];
+    }
+    __syncthreads();
+    const bool first = tid < nr && (tid == 0 || rank_bin[tid - 1] != bin);
+    uint32_t n_seg, total;
+    const uint32_t id = block_scan<kMapThreads>(first ? 1u : 0u, waves, &n_seg);
+    if (first) seg_rank[id] = static_cast<uint32_t>(tid);
+    if (tid == 0) seg_rank[n_seg] = static_cast<uint32_t>(nr);
+    const uint32_t count = first ? h[bin] : 0u;
+    const uint32_t off = block_scan<kMapThreads>(count, waves, &total);
+    // (the counts cover the tensor unless something wrote to it meanwhile)
+    const bool fits = all == static_cast<uint32_t>(T.n) && total <= T.cand_cap;
+    if (__syncthreads_or(!fits || count > kSegMax)) {
+        if (tid == 0) a.state[t] = kRadix;
+        return;
+    }
+    bool few_seg = false;
+    if (first) {
+        Segment s;
+        s.first = T.cand_first + off;
+        s.count = count;
+        s.rank_first = T.rank_first + tid;
+        s.n_ranks = seg_rank[id + 1] - static_cast<uint32_t>(tid);
+        s.tensor = t;
+        const bool in0 = hbin[0] == bin, in1 = hbin[1] == bin;
+        s.n_heavy = (in0 ? 1 : 0) + (in1 ? 1 : 0);
+        s.heavy_key[0] = in0 ? T.heavy_key[0] : T.heavy_key[1];
+        s.heavy_count[0] = in0 ? T.heavy_count[0] : T.heavy_count[1];
+        s.heavy_key[1] = T.heavy_key[1];
+        s.heavy_count[1] = T.heavy_count[1];
+        a.seg[T.rank_first + id] = s;
+        few_seg = few(s);
+        wanted[bin] = static_cast<uint16_t>(id + 1);
+    }
+    // onto the select kernels' lists, one add per list (adds of all segments to
+    // one address took 260 us for 26,000 of them)
+    uint32_t n_few_here;
+    const uint32_t at_few = block_scan<kMapThreads>(few_seg ? 1u : 0u, waves, &n_few_here);
+    if (tid == 0) {
+        hbin[0] = atomicAdd(&a.n_few[0], n_few_here);
+        hbin[1] = atomicAdd(&a.n_few[1], n_seg - n_few_here);
+    }
+    __syncthreads();
+    if (first) {
+        if (few_seg) a.few[hbin[0] + at_few] = T.rank_first + id;
+        else a.many[hbin[1] + id - at_few] = T.rank_first + id;
+    }
+}
+
+struct CollectOp {
+    uint32_t *stage;
+    uint32_t *s_count;
+    const uint2 *cell;
+    const uint16_t *want;         // 1 + segment, or 0
+    Map map;
+    uint32_t n_heavy, hk0, hk1;
+    // where candidates go past a full stage
+    const Segment *seg;
+    uint32_t *cursor, *cand;
+    uint32_t *place;              // staged candidates of each segment
+    __device__ __forceinline__ uint32_t segment(uint32_t key) const { return want[map.bin(key, cell)] - 1u; }
+    // candidate to place `at` of its segment (never past the segment's end)
+    __device__ __forceinline__ void put(uint32_t s, uint32_t at, uint32_t key) const {
+        if (at < seg[s].count) cand[seg[s].first + at] = key;
+    }
+    // a wave's candidates past a full stage (`mine`: this lane has one; all
+    // lanes take part): crowded, so mostly of one segment, one add for each
+    __device__ __forceinline__ void spill(bool mine, uint32_t key) const {
+        const uint32_t s = mine ? segment(key) : 0u;
+        while (true) {
+            const uint64_t todo = __ballot(mine);
+            if (todo == 0) break;
+            const int lead = __ffsll(static_cast<unsigned long long>(todo)) - 1;
+            const bool same = mine && s == static_cast<uint32_t>(__shfl(s, lead, 64));
+            const uint64_t m = __ballot(same);
+            uint32_t base = 0;
+            if (static_cast<int>(threadIdx.x & 63) == lead) base = atomicAdd(&cursor[s], static_cast<uint32_t>(__popcll(m)));
+            base = __shfl(base, lead, 64);
+            if (same) {
+                const uint64_t below = m & ((1ull << (threadIdx.x & 63)) - 1);
+                put(s, base + static_cast<uint32_t>(__popcll(below)), key);
+                mine = false;
+            }
+        }
+    }
+    template <bool PLAIN, int N, int V>
+    __device__ __forceinline__ void vecs(const uint32_t (&bits)[N], const bool (&in)[V]) {
+        uint32_t b[N];
+        if (PLAIN) {
+#pragma unroll
+            for (int e = 0; e < N; ++e) b[e] = map.bin_of_bits(bits[e], cell);
+        } else {
+#pragma unroll
+            for (int e = 0; e < N; ++e) b[e] = map.bin(key_of(bits[e]), cell);
+        }
+        bool w[N];
+        uint32_t to[N];
+#pragma unroll
+        for (int e = 0; e < N; ++e) {
+            to[e] = want[b[e]];
+            w[e] = to[e] != 0 && (PLAIN || in[e >> 2]);
+        }
+        if (n_heavy) {
+#pragma unroll
+            for (int e = 0; e < N; ++e) w[e] = w[e] && key_of(bits[e]) != hk0 && key_of(bits[e]) != hk1;
+        }
+        uint32_t mine = 0;
+#pragma unroll
+        for (int e = 0; e < N; ++e) mine += w[e] ? 1u : 0u;
+        if (__ballot(mine != 0) == 0) return;
+        // this thread's candidates: the next `mine` places of the stage.  (An
+        // index the compiler cannot see to be zero: for one address it would
+        // first add up the lanes' counts one by one, which took longer than the
+        // rest of the loop.)
+        uint32_t zero;
+        asm("v_mov_b32 %0, 0" : "=v"(zero));
+        uint32_t at = mine ? atomicAdd(s_count + zero, mine) : 0u;
+        if (__ballot(at + mine > static_cast<uint32_t>(kStage)) == 0) {
+#pragma unroll
+            for (int e = 0; e < N; ++e)
+                if (w[e]) {
+                    stage[at++] = bits[e];
+                    atomicAdd(&place[to[e] - 1u], 1u);
+                }
+        } else {
+            // not unrolled (rare, and its registers would cost the fast path its
+            // occupancy): the values move down one place each turn
+            uint32_t left = 0, q[N];
+#pragma unroll
+            for (int e = 0; e < N; ++e) {
+                left |= w[e] ? 1u << e : 0u;
+                q[e] = bits[e];
+            }
+#pragma clang loop unroll(disable)
+            while (__ballot(left != 0) != 0) {
+                const bool full = (left & 1u) && at >= static_cast<uint32_t>(kStage);
+                if ((left & 1u) && !full) {
+                    stage[at] = q[0];
+                    atomicAdd(&place[segment(key_of(q[0]))], 1u);
+                }
+                at += left & 1u;
+                spill(full, key_of(q[0]));
+                left >>= 1;
+#pragma unroll
+                for (int e = 0; e + 1 < N; ++e) q[e] = q[e + 1];
+            }
+        }
+    }
+    __device__ __forceinline__ void single(uint32_t bits, bool in) {
+        const uint32_t key = key_of(bits);
+        const bool w = in && !(n_heavy && (key == hk0 || key == hk1)) && want[map.bin(key, cell)] != 0;
+        const uint32_t at = w ? atomicAdd(s_count, 1u) : 0u;
+        if (w && at < static_cast<uint32_t>(kStage)) {
+            stage[at] = bits;
+            atomicAdd(&place[segment(key)], 1u);
+        }
+        spill(w && at >= static_cast<uint32_t>(kStage), key);
+    }
+};
+
+__global__ __launch_bounds__(kCollectThreads) void sampled_collect_kernel(Args a) {
+    __shared__ uint2 cell[kCells];
+    __shared__ uint16_t want[kMaxBins];
+    __shared__ uint32_t stage[kStage];
+    __shared__ uint32_t place[kMaxRanks];            // flush: candidates of each segment, then where they go
+    __shared__ uint32_t s_count;
+    constexpr uint32_t kNowhere = 0x80000000u;       // (a tensor's candidates are fewer)
+    const Tile tile = a.tile[blockIdx.x];
+    const Tensor &T = a.tensor[tile.tensor];
+    if (a.state[tile.tensor] != kRun) return;
+    const int tid = threadIdx.x;
+    const uint32_t bins = T.bins;
+    const uint16_t *wanted = a.wanted + static_cast<int64_t>(T.bin_first);
+    for (int i = tid; i < kCells; i += kCollectThreads) cell[i] = a.cell[static_cast<int64_t>(T.map) * kCells + i];
+    for (uint32_t i = tid; i < bins; i += kCollectThreads) want[i] = wanted[i];
+    const int nr = T.n_ranks;
+    for (int i = tid; i < nr; i += kCollectThreads) place[i] = 0;
+    if (tid == 0) s_count = 0;
+    __syncthreads();
+    const Map map{T.key0, T.shift};
+    const uint32_t nh = T.n_heavy;
+    CollectOp op{stage, &s_count, cell, want, map, nh, T.heavy_key[0], T.heavy_key[nh > 1 ? 1 : 0],
+                 a.seg + T.rank_first, a.cursor + T.rank_first, a.cand, place};
+    uint32_t *cand = a.cand + T.cand_first;
+    // Staged candidates, counted per segment as they come, go out once they fill
+    // most of the stage: room taken with one global add per segment, then each to its
+    // place.  (A stage that fills up between two looks, where the wanted values
+    // are crowded, as in sorted data, sends the rest out one by one.)  On 1.3G
+    // values the reads and the staging take 810 us, this 450 more: 4-byte writes
+    // to some 190 places per flush.
+    for_values<kCollectThreads, 2>(T.x, T.n, tile.first, tile.last, map.takes_bits(), op, [&](bool last) {
+        __syncthreads();
+        const uint32_t asked = s_count;
+        __syncthreads();                                         // read by all before the next iteration adds to it
+        if (asked < 6 * kStage / 10 && !last) return;            // uniform
+        const uint32_t count = min(asked, static_cast<uint32_t>(kStage));
+        for (int i = tid; i < nr; i += kCollectThreads) {
+            const uint32_t m = place[i];
+            if (m) {
+                const uint32_t at = atomicAdd(&op.cursor[i], m);
+                // (past its end only if something wrote to the tensor meanwhile)
+                place[i] = at + m <= op.seg[i].count ? static_cast<uint32_t>(op.seg[i].first - T.cand_first) + at : kNowhere;
+            }
+        }
+        __syncthreads();
+        for (uint32_t i = tid; i < count; i += kCollectThreads) {
+            const uint32_t key = key_of(stage[i]), s = op.segment(key);
+            if (place[s] < kNowhere) cand[atomicAdd(&place[s], 1u)] = key;
+        }
+        __syncthreads();
+        for (int i = tid; i < nr; i += kCollectThreads) place[i] = 0;
+        if (tid == 0) s_count = 0;
+        __syncthreads();
+    });
+}
+
+// A rank within its segment -> its rank among the candidates, or the repeated
+// key it falls on (true).  less[q]: candidates below repeated key q.
+__device__ __forceinline__ bool on_heavy(const Segment &s, const uint32_t *less, uint32_t &r, uint32_t &key) {
+    if (s.n_heavy == 0) return false;
+    // at most two, taken in key order
+    const bool swap = s.n_heavy > 1 && s.heavy_key[1] < s.heavy_key[0];
+    const uint32_t l0 = swap ? less[1] : less[0], c0 = swap ? s.heavy_count[1] : s.heavy_count[0];
+    if (r < l0) return false;
+    if (r < l0 + c0) {
+        key = swap ? s.heavy_key[1] : s.heavy_key[0];
+        return true;
+    }
+    r -= c0;
+    if (s.n_heavy == 1) return false;
+    const uint32_t l1 = swap ? less[0] : less[1], c1 = swap ? s.heavy_count[0] : s.heavy_count[1];
+    if (r < l1) return false;
+    if (r < l1 + c1) {
+        key = swap ? s.heavy_key[0] : s.heavy_key[1];
+        return true;
+    }
+    r -= c1;
+    return false;
+}
+
+// Calls f(i, p[i]) for every i < n, four loads in flight per thread.
+template <int NT, typename F>
+__device__ __forceinline__ void each_key(const uint32_t *p, uint32_t n, F f) {
+    uint32_t i = threadIdx.x;
+    for (; i + 3 * NT < n; i += 4 * NT) {
+        uint32_t k[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) k[u] = p[i + u * NT];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) f(i + u * NT, k[u]);
+    }
+    for (; i < n; i += NT) f(i, p[i]);
+}
+
+constexpr int kDigitBins = 1 << kSegDigit;
+
+// Shift that takes a range of `width` + 1 keys to at most 2^bits parts.
+__device__ __forceinline__ int part_shift(uint32_t width, int bits) {
+    return width ? max(0, 32 - __builtin_clz(width) - bits) : 0;
+}
+
+// The r-th smallest of a segment's candidates, whose keys lie in [lo, hi]:
+// digits of 11 bits of the segment's own range (one or two, as a bin spans few
+// keys).  each(f) calls f(key) for every candidate, spread over the threads.
+template <int NT, typename E>
+__device__ __forceinline__ uint32_t select_rank(uint32_t r, uint32_t lo, uint32_t hi, uint32_t *h, uint32_t *waves,
+                                                uint32_t *digit, E each) {
+    uint32_t from = lo, width = hi - lo;             // the rank is among the keys [from, from + width]
+    while (width) {
+        const int sh = part_shift(width, kSegDigit);
+        __syncthreads();
+        for (int i = threadIdx.x; i < kDigitBins; i += NT) h[i] = 0;
+        __syncthreads();
+        each([&](uint32_t k) {
+            const uint32_t d = k - from;
+            if (d <= width) atomicAdd(&h[d >> sh], 1u);
+        });
+        __syncthreads();
+        constexpr int kPerT = kDigitBins / NT;
+        uint32_t c[kPerT], sum = 0, all;
+#pragma unroll
+        for (int k = 0; k < kPerT; ++k) sum += c[k] = h[threadIdx.x * kPerT + k];
+        uint32_t before = block_scan<NT>(sum, waves, &all);
+#pragma unroll
+        for (int k = 0; k < kPerT; ++k) {
+            if (r >= before && r < before + c[k]) {
+                digit[0] = static_cast<uint32_t>(threadIdx.x * kPerT + k);
+                digit[1] = r - before;
+            }
+            before += c[k];
+        }
+        __syncthreads();
+        const uint32_t d = digit[0];
+        r = digit[1];
+        width = sh ? min((1u << sh) - 1u, width - (d << sh)) : 0u;
+        from += d << sh;
+    }
+    return from;
+}
+
+// One workgroup per wanted bin of at most 4 ranks and 4,096 candidates: nearly
+// all of them.  The candidates are read once, into registers.
+__global__ __launch_bounds__(kSmallThreads) void segment_few_kernel(Args a) {
+    __shared__ uint32_t h[kDigitBins];
+    __shared__ uint32_t waves[kSmallThreads / 64];
+    __shared__ uint32_t s_lo, s_hi, s_less[kHeavy], s_digit[2];
+    const int tid = threadIdx.x;
+    const uint32_t n = a.n_few[0];
+    for (uint32_t slot = blockIdx.x; slot < n; slot += gridDim.x) {
+    const Segment s = a.seg[a.few[slot]];
+    __syncthreads();                                 // s_lo and the others are read by the segment before
+    const uint32_t *p = a.cand + s.first;
+    if (tid == 0) {
+        s_lo = 0xffffffffu;
+        s_hi = 0;
+        s_less[0] = s_less[1] = 0;
+    }
+    uint32_t key[kSmallPer];
+    uint32_t mn = 0xffffffffu, mx = 0, l0 = 0, l1 = 0;
+#pragma unroll
+    for (int u = 0; u < kSmallPer; ++u) {
+        const uint32_t i = tid + u * kSmallThreads;
+        key[u] = i < s.count ? p[i] : 0u;
+    }
+#pragma unroll
+    for (int u = 0; u < kSmallPer; ++u) {
+        if (tid + u * kSmallThreads < s.count) {
+            mn = min(mn, key[u]);
+            mx = max(mx, key[u]);
+            l0 += s.n_heavy > 0 && key[u] < s.heavy_key[0];
+            l1 += s.n_heavy > 1 && key[u] < s.heavy_key[1];
+        }
+    }
+    mn = wave_min(mn);
+    mx = wave_max(mx);
+    __syncthreads();
+    if ((tid & 63) == 0) {
+        atomicMin(&s_lo, mn);
+        atomicMax(&s_hi, mx);
+    }
+    if (s.n_heavy) {
+        if (l0) atomicAdd(&s_less[0], l0);
+        if (l1) atomicAdd(&s_less[1], l1);
+    }
+    __syncthreads();
+    const uint32_t lo = s_lo, hi = s_hi, less[kHeavy] = {s_less[0], s_less[1]};
+    for (uint32_t j = 0; j < s.n_ranks; ++j) {
+        uint32_t r = a.residual[s.rank_first + j], k = lo;
+        if (!on_heavy(s, less, r, k) && s.count)
+            k = select_rank<kSmallThreads>(r, lo, hi, h, waves, s_digit, [&](auto f) {
+#pragma unroll
+                for (int u = 0; u < kSmallPer; ++u)
+                    if (tid + u * kSmallThreads < s.count) f(key[u]);
+            });
+        if (tid == 0) a.out[s.rank_first + j] = key_bits(k);
+    }
+    }
+}
+
+// The other segments: large bins, and the outer bins, which hold the extreme
+// ranks.  Up to 4 ranks: one by one, as above.  More: up to 4,096 candidates are
+// sorted in LDS; past that a histogram of 8,192 equal parts of their range tells
+// the parts that hold ranks, whose candidates are sorted group by group (a sort
+// of 8,192 keys takes about 36 us: with 2,048 parts, and segments of up to 8,192
+// candidates sorted whole, the two outer bins of a tensor of 30M uniform values
+// took 190 us, now 150).  A part too large for that becomes a range of its own.
+__global__ __launch_bounds__(kSegThreads) void segment_many_kernel(Args a) {
+    constexpr int kRanges = 32;
+    constexpr int kParts = 1 << kPartBits;
+    constexpr uint32_t kGroup = kSegSort / 2;        // a part at most, and a group's wanted candidates but the last part
+    constexpr uint32_t kNot = 0xffffffffu;
+    __shared__ uint32_t h[kParts];
+    __shared__ uint32_t x[kSegSort];
+    __shared__ uint32_t place[kMaxRanks];            // 2 * a rank's place among the candidates, + 1: it is a repeated key's
+    __shared__ uint32_t waves[kSegThreads / 64];
+    __shared__ uint32_t s_lo, s_hi, s_less[kHeavy], s_digit[2], s_n;
+    __shared__ uint32_t r_from[kRanges], r_width[kRanges], r_base[kRanges], n_range, s_fail;
+    const int tid = threadIdx.x;
+    const uint32_t n = a.n_few[1];
+    for (uint32_t slot = blockIdx.x; slot < n; slot += gridDim.x) {
+    const Segment s = a.seg[a.many[slot]];
+    __syncthreads();                                 // LDS is read by the segment before
+    const uint32_t *p = a.cand + s.first;
+    if (tid == 0) {
+        s_lo = 0xffffffffu;
+        s_hi = 0;
+        s_less[0] = s_less[1] = 0;
+        s_fail = 0;
+    }
+    __syncthreads();
+    uint32_t mn = 0xffffffffu, mx = 0, l0 = 0, l1 = 0;
+    each_key<kSegThreads>(p, s.count, [&](uint32_t, uint32_t k) {
+        mn = min(mn, k);
+        mx = max(mx, k);
+        l0 += s.n_heavy > 0 && k < s.heavy_key[0];
+        l1 += s.n_heavy > 1 && k < s.heavy_key[1];
+    });
+    mn = wave_min(mn);
+    mx = wave_max(mx);
+    if ((tid & 63) == 0) {
+        atomicMin(&s_lo, mn);
+        atomicMax(&s_hi, mx);
+    }
+    if (s.n_heavy) {
+        if (l0) atomicAdd(&s_less[0], l0);
+        if (l1) atomicAdd(&s_less[1], l1);
+    }
+    __syncthreads();
+    const uint32_t lo = s_lo, hi = s_hi, less[kHeavy] = {s_less[0], s_less[1]};
+    if (s.n_ranks <= 4) {
+        for (uint32_t j = 0; j < s.n_ranks; ++j) {
+            uint32_t r = a.residual[s.rank_first + j], k = lo;
+            if (!on_heavy(s, less, r, k) && s.count)
+                k = select_rank<kSegThreads>(r, lo, hi, h, waves, s_digit, [&](auto f) {
+                    each_key<kSegThreads>(p, s.count, [&](uint32_t, uint32_t key) { f(key); });
+                });
+            if (tid == 0) a.out[s.rank_first + j] = key_bits(k);
+        }
+        continue;
+    }
+    for (uint32_t j = tid; j < s.n_ranks; j += kSegThreads) {
+        uint32_t r = a.residual[s.rank_first + j], k;
+        const bool rep = on_heavy(s, less, r, k);
+        if (rep) {
+            // (its place: the candidates below it, so that places stay in order)
+            r = s.n_heavy > 1 && k == s.heavy_key[1] ? less[1] : less[0];
+            a.out[s.rank_first + j] = key_bits(k);
+        }
+        place[j] = 2 * r + (rep ? 1u : 0u);
+    }
+    if (s.count == 0) continue;
+    if (s.count <= static_cast<uint32_t>(kSegSort)) {
+        const int pw = pow2_at_least(s.count);
+        for (uint32_t i = tid; i < static_cast<uint32_t>(pw); i += kSegThreads) x[i] = i < s.count ? p[i] : 0xffffffffu;
+        lds_sort<kSegThreads>(x, pw);                // (its first step waits for place too)
+        for (uint32_t j = tid; j < s.n_ranks; j += kSegThreads)
+            if (!(place[j] & 1u)) a.out[s.rank_first + j] = key_bits(x[min(place[j] >> 1, s.count - 1)]);
+        continue;
+    }
+    if (tid == 0) {
+        r_from[0] = lo;
+        r_width[0] = hi - lo;
+        r_base[0] = 0;
+        n_range = 1;
+    }
+    __syncthreads();
+    // first rank (index into place) at or past candidate place c
+    auto first_at = [&](uint32_t c) {
+        uint32_t l = 0, u = s.n_ranks;
+        while (l < u) {
+            const uint32_t mid = (l + u) >> 1;
+            if ((place[mid] >> 1) < c) l = mid + 1; else u = mid;
+        }
+        return l;
+    };
+    while (true) {
+        const uint32_t left = n_range;
+        __syncthreads();
+        if (left == 0 || s_fail) break;              // uniform
+        const uint32_t from = r_from[left - 1], width = r_width[left - 1], base = r_base[left - 1];
+        for (int i = tid; i < kParts; i += kSegThreads) h[i] = 0;
+        __syncthreads();
+        if (tid == 0) n_range = left - 1;
+        const int sh = part_shift(width, kPartBits);
+        each_key<kSegThreads>(p, s.count, [&](uint32_t, uint32_t k) {
+            const uint32_t d = k - from;
+            if (d <= width) atomicAdd(&h[d >> sh], 1u);
+        });
+        __syncthreads();
+        constexpr int kPerT = kParts / kSegThreads;
+        uint32_t c[kPerT], sum = 0, all;
+#pragma unroll
+        for (int k = 0; k < kPerT; ++k) sum += c[k] = h[tid * kPerT + k];
+        const uint32_t start = base + block_scan<kSegThreads>(sum, waves, &all);
+        bool sorted[kPerT];
+        uint32_t before = start, want = 0;
+#pragma unroll
+        for (int k = 0; k < kPerT; ++k) {
+            const uint32_t j0 = first_at(before), j1 = first_at(before + c[k]);
+            sorted[k] = j1 > j0;
+            if (j1 > j0 && (sh == 0 || c[k] > kGroup)) {
+                // one key, or a range of its own
+                sorted[k] = false;
+                const uint32_t key = from + (static_cast<uint32_t>(tid * kPerT + k) << sh);
+                if (sh == 0) {
+                    for (uint32_t j = j0; j < j1; ++j)
+                        if (!(place[j] & 1u)) a.out[s.rank_first + j] = key_bits(key);
+                } else {
+                    const uint32_t at = atomicAdd(&n_range, 1u);
+                    if (at < kRanges) {
+                        r_from[at] = key;
+                        r_width[at] = min((1u << sh) - 1u, from + width - key);
+                        r_base[at] = before;
+                    } else {
+                        s_fail = 1;
+                    }
+                }
+            }
+            want += sorted[k] ? c[k] : 0u;
+            before += c[k];
+        }
+        uint32_t total;
+        uint32_t at = block_scan<kSegThreads>(want, waves, &total);
+        // h: a part's group (wanted candidates before it / kGroup)
+#pragma unroll
+        for (int k = 0; k < kPerT; ++k) {
+            h[tid * kPerT + k] = sorted[k] ? at / kGroup : kNot;
+            at += sorted[k] ? c[k] : 0u;
+        }
+        at -= want;
+        for (uint32_t g = 0; g * kGroup < total; ++g) {
+            if (tid == 0) s_n = 0;
+            __syncthreads();
+            each_key<kSegThreads>(p, s.count, [&](uint32_t, uint32_t k) {
+                const uint32_t d = k - from;
+                if (d <= width && h[d >> sh] == g) {
+                    const uint32_t e = atomicAdd(&s_n, 1u);
+                    if (e < static_cast<uint32_t>(kSegSort)) x[e] = k;
+                }
+            });
+            __syncthreads();
+            const uint32_t m = min(s_n, static_cast<uint32_t>(kSegSort));
+            const int pw = pow2_at_least(m);
+            for (uint32_t i = m + tid; i < static_cast<uint32_t>(pw); i += kSegThreads) x[i] = 0xffffffffu;
+            lds_sort<kSegThreads>(x, pw);
+            // each part's first candidate in the sorted group is where its keys begin
+            uint32_t b = start;
+#pragma unroll
+            for (int k = 0; k < kPerT; ++k) {
+                if (sorted[k] && h[tid * kPerT + k] == g && m) {
+                    const uint32_t key = from + (static_cast<uint32_t>(tid * kPerT + k) << sh);
+                    uint32_t l = 0, u = m;
+                    while (l < u) {
+                        const uint32_t mid = (l + u) >> 1;
+                        if (x[mid] < key) l = mid + 1; else u = mid;
+                    }
+                    for (uint32_t j = first_at(b); j < s.n_ranks && (place[j] >> 1) < b + c[k]; ++j)
+                        if (!(place[j] & 1u)) a.out[s.rank_first + j] = key_bits(x[min(l + (place[j] >> 1) - b, m - 1)]);
+                }
+                b += c[k];
+            }
+            __syncthreads();
+        }
+    }
+    if (s_fail && tid == 0) a.state[s.tensor] = kRadix;
+    }
+}
+
+// The big tensors (over kSortMax) of a call, as the workspace needs them.
+struct Sizes {
+    int64_t tensors = 0, ranks = 0;      // all that take this path
+    int64_t big = 0, tiles = 0, bins = 0;
+    uint64_t cand = 0;
+};
+
+struct Layout {
+    size_t tensor, tile, rank, n_few, upload_end;    // one upload
+    size_t residual, cell, hist, wanted, seg, cursor, few, many;
+    size_t out, state, cand, total;                  // out and state come back in one copy
+};
+
+// Elements of one tile of the reads: about kTilesWanted tiles in all.
+constexpr int64_t kTilesWanted = 4096;
+inline int64_t tile_elems(int64_t total) {
+    const int64_t t = (total / kTilesWanted + kHistIter - 1) / kHistIter * kHistIter;
+    return std::min<int64_t>(std::max<int64_t>(t, 2 * kHistIter), 1 << 20);
+}
+
+inline bool takes(int64_t n, int64_t ranks) { return n > 0 && n <= kMaxElems && ranks > 0 && ranks <= kMaxRanks; }
+
+// Bins of a tensor's map: enough that the wanted bins hold few of its values,
+// few enough that adding a tile's counts to the tensor's costs little.
+inline uint32_t bin_budget(int64_t n) { return n >= (1 << 21) ? 8192u : n >= (1 << 19) ? 4096u : 2048u; }
+
+inline Sizes sizes(const int64_t *numel, const int64_t *rank_first, int32_t n) {
+    Sizes z;
+    int64_t total = 0;
+    for (int32_t i = 0; i < n; ++i)
+        if (takes(numel[i], rank_first[i + 1] - rank_first[i]) && numel[i] > kSortMax) total += numel[i];
+    const int64_t tile = tile_elems(total);
+    for (int32_t i = 0; i < n; ++i) {
+        const int64_t r = rank_first[i + 1] - rank_first[i];
+        if (!takes(numel[i], r)) continue;
+        ++z.tensors;
+        z.ranks += r;
+        if (numel[i] <= kSortMax) continue;
+        ++z.big;
+        z.tiles += (numel[i] + tile - 1) / tile;
+        z.bins += bin_budget(numel[i]);
+        z.cand += static_cast<uint64_t>(numel[i]) / kCandDen;
+    }
+    return z;
+}
+
+inline Layout layout(const Sizes &z) {
+    auto up = [](size_t b) { return (b + 255) / 256 * 256; };
+    Layout L{};
+    size_t off = 0;
+    const size_t nt = static_cast<size_t>(z.tensors), nr = static_cast<size_t>(z.ranks);
+    L.tensor = off; off += up(sizeof(Tensor) * nt);
+    L.tile = off; off += up(sizeof(Tile) * static_cast<size_t>(z.tiles));
+    L.rank = off; off += up(4 * nr);
+    L.n_few = off; off += 256;
+    L.upload_end = off;
+    L.residual = off; off += up(4 * nr);
+    L.cell = off; off += up(sizeof(uint2) * kCells * static_cast<size_t>(z.big));
+    L.hist = off; off += up(4 * static_cast<size_t>(z.bins));
+    L.wanted = off; off += up(2 * static_cast<size_t>(z.bins));
+    L.seg = off; off += up(sizeof(Segment) * nr);
+    L.cursor = off; off += up(4 * nr);
+    L.few = off; off += up(4 * nr);
+    L.many = off; off += up(4 * nr);
+    L.out = off; off += 4 * nr;
+    L.state = off; off += up(4 * nt);
+    L.cand = off; off += up(4 * static_cast<size_t>(z.cand));
+    L.total = off;
+    return L;
+}
+
+}  // namespace sampled

@@ -40,6 +40,7 @@
 #include <cstdint>
 #include <cstdio>
 #include <cstring>
+#include <type_traits>
 #include <vector>
 
 #include "adana_mta.h"
@@ -448,6 +449,33 @@ void tile_layout(const int64_t *numel, const int64_t *rank_first, int32_t n, std
     }
 }
 
+// The argument checks of both selects.
+int check_request(const char *fn, const float *const *h_tensor, const int64_t *h_numel, int32_t n,
+                  const int64_t *h_ranks, const int64_t *h_rank_first, const float *h_values) {
+    if (n < 0 || (n > 0 && (!h_tensor || !h_numel || !h_rank_first)))
+        return adana_set_error(ADANA_E_INVALID, "%s: bad arguments", fn);
+    if (n == 0) return ADANA_OK;
+    const int64_t total = h_rank_first[n];
+    if (total < 0 || (total > 0 && (!h_ranks || !h_values)))
+        return adana_set_error(ADANA_E_INVALID, "%s: bad rank arrays", fn);
+    for (int32_t i = 0; i < n; ++i) {
+        if (h_numel[i] < 0 || h_rank_first[i] > h_rank_first[i + 1] || h_rank_first[i] < 0)
+            return adana_set_error(ADANA_E_INVALID, "%s: bad sizes at tensor %d", fn, i);
+        if (h_numel[i] > 0xffffffffLL)          // histogram bins are 32-bit counters
+            return adana_set_error(ADANA_E_UNSUPPORTED, "%s: tensor %d has %lld elements (at most 2^32 - 1)",
+                                   fn, i, static_cast<long long>(h_numel[i]));
+        if (h_rank_first[i + 1] > h_rank_first[i] && !h_tensor[i])
+            return adana_set_error(ADANA_E_INVALID, "%s: null tensor %d", fn, i);
+        for (int64_t j = h_rank_first[i]; j < h_rank_first[i + 1]; ++j)
+            if (h_ranks[j] < 0 || h_ranks[j] >= h_numel[i])
+                return adana_set_error(ADANA_E_INVALID, "%s: rank %lld outside tensor %d of %lld elements",
+                            fn, static_cast<long long>(h_ranks[j]), i, static_cast<long long>(h_numel[i]));
+    }
+    return ADANA_OK;
+}
+
+#include "adana_order_sampled.h"
+
 }  // namespace
 
 extern "C" {
@@ -470,25 +498,9 @@ size_t adana_order_stats_workspace_compact(const int64_t *h_numel, const int64_t
 int adana_order_stats(const float *const *h_tensor, const int64_t *h_numel, int32_t n,
                       const int64_t *h_ranks, const int64_t *h_rank_first, float *h_values,
                       void *d_workspace, size_t ws_bytes, void *stream) {
-    if (n < 0 || (n > 0 && (!h_tensor || !h_numel || !h_rank_first)))
-        return adana_set_error(ADANA_E_INVALID, "adana_order_stats: bad arguments");
-    if (n == 0) return ADANA_OK;
+    const int valid = check_request("adana_order_stats", h_tensor, h_numel, n, h_ranks, h_rank_first, h_values);
+    if (valid != ADANA_OK || n == 0) return valid;
     const int64_t total = h_rank_first[n];
-    if (total < 0 || (total > 0 && (!h_ranks || !h_values)))
-        return adana_set_error(ADANA_E_INVALID, "adana_order_stats: bad rank arrays");
-    for (int32_t i = 0; i < n; ++i) {
-        if (h_numel[i] < 0 || h_rank_first[i] > h_rank_first[i + 1] || h_rank_first[i] < 0)
-            return adana_set_error(ADANA_E_INVALID, "adana_order_stats: bad sizes at tensor %d", i);
-        if (h_numel[i] > 0xffffffffLL)          // histogram bins are 32-bit counters
-            return adana_set_error(ADANA_E_UNSUPPORTED, "adana_order_stats: tensor %d has %lld elements (at most 2^32 - 1)",
-                                   i, static_cast<long long>(h_numel[i]));
-        if (h_rank_first[i + 1] > h_rank_first[i] && !h_tensor[i])
-            return adana_set_error(ADANA_E_INVALID, "adana_order_stats: null tensor %d", i);
-        for (int64_t j = h_rank_first[i]; j < h_rank_first[i + 1]; ++j)
-            if (h_ranks[j] < 0 || h_ranks[j] >= h_numel[i])
-                return adana_set_error(ADANA_E_INVALID, "adana_order_stats: rank %lld outside tensor %d of %lld elements",
-                            static_cast<long long>(h_ranks[j]), i, static_cast<long long>(h_numel[i]));
-    }
     if (total == 0) return ADANA_OK;
     std::vector<int64_t> tile_first;
     tile_layout(h_numel, h_rank_first, n, tile_first);
@@ -663,6 +675,157 @@ int adana_order_stats(const float *const *h_tensor, const int64_t *h_numel, int3
         const uint32_t b = key_to_bits(rank_prefix[j]);
         memcpy(&h_values[j], &b, 4);
     }
+    return ADANA_OK;
+}
+
+size_t adana_order_stats_sampled_workspace(const int64_t *h_numel, const int64_t *h_rank_first, int32_t n_tensors) {
+    const size_t radix = adana_order_stats_workspace_compact(h_numel, h_rank_first, n_tensors);
+    if (radix == 0 || n_tensors == 0) return radix;
+    return std::max(radix, sampled::layout(sampled::sizes(h_numel, h_rank_first, n_tensors)).total);
+}
+
+int adana_order_stats_sampled(const float *const *h_tensor, const int64_t *h_numel, int32_t n,
+                              const int64_t *h_ranks, const int64_t *h_rank_first, float *h_values,
+                              void *d_workspace, size_t ws_bytes, void *stream) {
+    const char *fn = "adana_order_stats_sampled";
+    const int valid = check_request(fn, h_tensor, h_numel, n, h_ranks, h_rank_first, h_values);
+    if (valid != ADANA_OK || n == 0) return valid;
+    if (h_rank_first[n] == 0) return ADANA_OK;
+    const size_t need = adana_order_stats_sampled_workspace(h_numel, h_rank_first, n);
+    if (!d_workspace || ws_bytes < need)
+        return adana_set_error(ADANA_E_INVALID, "%s: workspace of %zu bytes < %zu needed", fn, ws_bytes, need);
+    const sampled::Sizes z = sampled::sizes(h_numel, h_rank_first, n);
+    const sampled::Layout L = sampled::layout(z);
+    char *ws = static_cast<char *>(d_workspace);
+    hipStream_t st = static_cast<hipStream_t>(stream);
+
+    // the tensors that take this path, their tiles and ascending ranks, as
+    // uploaded; order[j]: where rank j's value goes
+    std::vector<char> up(L.upload_end);
+    sampled::Tensor *ten = reinterpret_cast<sampled::Tensor *>(up.data() + L.tensor);
+    sampled::Tile *tile = reinterpret_cast<sampled::Tile *>(up.data() + L.tile);
+    uint32_t *rank = reinterpret_cast<uint32_t *>(up.data() + L.rank);
+    std::vector<int32_t> taken, radix;
+    std::vector<int64_t> order(static_cast<size_t>(z.ranks));
+    int64_t big_total = 0;
+    for (int32_t i = 0; i < n; ++i) {
+        const int64_t r = h_rank_first[i + 1] - h_rank_first[i];
+        if (sampled::takes(h_numel[i], r)) {
+            taken.push_back(i);
+            if (h_numel[i] > sampled::kSortMax) big_total += h_numel[i];
+        } else if (r > 0) {
+            radix.push_back(i);
+        }
+    }
+    const int64_t per_tile = sampled::tile_elems(big_total);
+    int64_t n_rank = 0, n_tile = 0, n_big = 0, n_bin = 0, max_bins = 0;
+    uint64_t n_cand = 0;
+    for (size_t k = 0; k < taken.size(); ++k) {
+        const int32_t i = taken[k];
+        const int64_t a = h_rank_first[i], b = h_rank_first[i + 1];
+        sampled::Tensor &t = ten[k];
+        t = sampled::Tensor{};
+        t.x = h_tensor[i];
+        t.n = static_cast<uint64_t>(h_numel[i]);
+        t.rank_first = static_cast<int32_t>(n_rank);
+        t.n_ranks = static_cast<int32_t>(b - a);
+        for (int64_t j = a; j < b; ++j) order[n_rank + j - a] = j;
+        if (!std::is_sorted(h_ranks + a, h_ranks + b))
+            std::sort(order.begin() + n_rank, order.begin() + n_rank + (b - a),
+                      [&](int64_t p, int64_t q) { return h_ranks[p] < h_ranks[q]; });
+        for (int64_t j = 0; j < b - a; ++j) rank[n_rank + j] = static_cast<uint32_t>(h_ranks[order[n_rank + j]]);
+        n_rank += b - a;
+        if (h_numel[i] <= sampled::kSortMax) continue;
+        t.cand_first = n_cand;
+        t.cand_cap = t.n / sampled::kCandDen;
+        n_cand += t.cand_cap;
+        t.bin_budget = sampled::bin_budget(h_numel[i]);
+        t.bin_first = static_cast<uint32_t>(n_bin);
+        n_bin += t.bin_budget;
+        max_bins = std::max<int64_t>(max_bins, t.bin_budget);
+        t.map = static_cast<uint32_t>(n_big++);
+        for (int64_t e = 0; e < h_numel[i]; e += per_tile)
+            tile[n_tile++] = sampled::Tile{static_cast<int32_t>(k), 0, static_cast<uint64_t>(e),
+                                           static_cast<uint64_t>(std::min(e + per_tile, h_numel[i]))};
+    }
+    if (n_rank > 0x7fffffffLL || n_tile > 0x7fffffffLL || n_bin > 0xffffffffLL)
+        return adana_set_error(ADANA_E_UNSUPPORTED, "%s: list too large", fn);
+    auto status = [fn](hipError_t e, const char *what) {
+        return e == hipSuccess ? static_cast<int>(ADANA_OK)
+                               : adana_set_error(ADANA_E_HIP, "%s: %s: %s", fn, what, hipGetErrorString(e));
+    };
+    int rc;
+    if (!taken.empty()) {
+        sampled::Args a{};
+        a.tensor = reinterpret_cast<sampled::Tensor *>(ws + L.tensor);
+        a.tile = reinterpret_cast<const sampled::Tile *>(ws + L.tile);
+        a.rank = reinterpret_cast<const uint32_t *>(ws + L.rank);
+        a.residual = reinterpret_cast<uint32_t *>(ws + L.residual);
+        a.cell = reinterpret_cast<uint2 *>(ws + L.cell);
+        a.hist = reinterpret_cast<uint32_t *>(ws + L.hist);
+        a.wanted = reinterpret_cast<uint16_t *>(ws + L.wanted);
+        a.seg = reinterpret_cast<sampled::Segment *>(ws + L.seg);
+        a.cursor = reinterpret_cast<uint32_t *>(ws + L.cursor);
+        a.few = reinterpret_cast<uint32_t *>(ws + L.few);
+        a.many = reinterpret_cast<uint32_t *>(ws + L.many);
+        a.n_few = reinterpret_cast<uint32_t *>(ws + L.n_few);
+        a.out = reinterpret_cast<uint32_t *>(ws + L.out);
+        a.state = reinterpret_cast<uint32_t *>(ws + L.state);
+        a.cand = reinterpret_cast<uint32_t *>(ws + L.cand);
+        a.n = static_cast<int32_t>(taken.size());
+        if ((rc = status(hipMemcpyAsync(ws, up.data(), up.size(), hipMemcpyHostToDevice, st), "copy"))) return rc;
+        const unsigned nt = static_cast<unsigned>(taken.size());
+        hipLaunchKernelGGL(sampled::sample_map_kernel, dim3(nt), dim3(sampled::kMapThreads), 0, st, a);
+        if ((rc = status(hipGetLastError(), "map launch"))) return rc;
+        if (n_tile > 0) {
+            const unsigned lds = static_cast<unsigned>(sizeof(uint2) * sampled::kCells + 4 * max_bins);
+            hipLaunchKernelGGL(sampled::sampled_hist_kernel, dim3(static_cast<unsigned>(n_tile)),
+                               dim3(sampled::kHistThreads), lds, st, a);
+            if ((rc = status(hipGetLastError(), "histogram launch"))) return rc;
+            hipLaunchKernelGGL(sampled::sampled_walk_kernel, dim3(nt), dim3(sampled::kMapThreads), 0, st, a);
+            if ((rc = status(hipGetLastError(), "walk launch"))) return rc;
+            hipLaunchKernelGGL(sampled::sampled_collect_kernel, dim3(static_cast<unsigned>(n_tile)),
+                               dim3(sampled::kCollectThreads), 0, st, a);
+            if ((rc = status(hipGetLastError(), "collect launch"))) return rc;
+            // a few workgroups per CU go through the lists that the walk left
+            hipLaunchKernelGGL(sampled::segment_few_kernel,
+                               dim3(static_cast<unsigned>(std::min<int64_t>(n_rank, sampled::kFewGrid))),
+                               dim3(sampled::kSmallThreads), 0, st, a);
+            if ((rc = status(hipGetLastError(), "select launch"))) return rc;
+            hipLaunchKernelGGL(sampled::segment_many_kernel,
+                               dim3(static_cast<unsigned>(std::min<int64_t>(n_rank, sampled::kManyGrid))),
+                               dim3(sampled::kSegThreads), 0, st, a);
+            if ((rc = status(hipGetLastError(), "select launch"))) return rc;
+        }
+        std::vector<uint32_t> back(static_cast<size_t>(n_rank) + taken.size());
+        if ((rc = status(hipMemcpyAsync(back.data(), ws + L.out, 4 * back.size(), hipMemcpyDeviceToHost, st), "copy")) ||
+            (rc = status(hipStreamSynchronize(st), "synchronize")))
+            return rc;
+        for (size_t k = 0; k < taken.size(); ++k) {
+            if (back[n_rank + k] == sampled::kRadix) {
+                radix.push_back(taken[k]);
+                continue;
+            }
+            for (int32_t j = ten[k].rank_first; j < ten[k].rank_first + ten[k].n_ranks; ++j)
+                memcpy(&h_values[order[j]], &back[j], 4);
+        }
+    }
+    if (radix.empty()) return ADANA_OK;
+    // the rest through the radix select, over the same workspace
+    std::vector<const float *> rt;
+    std::vector<int64_t> rn, rr, rf{0};
+    for (const int32_t i : radix) {
+        rt.push_back(h_tensor[i]);
+        rn.push_back(h_numel[i]);
+        rr.insert(rr.end(), h_ranks + h_rank_first[i], h_ranks + h_rank_first[i + 1]);
+        rf.push_back(static_cast<int64_t>(rr.size()));
+    }
+    std::vector<float> rv(rr.size());
+    if ((rc = adana_order_stats(rt.data(), rn.data(), static_cast<int32_t>(radix.size()), rr.data(), rf.data(),
+                                rv.data(), d_workspace, ws_bytes, stream)))
+        return rc;
+    for (size_t k = 0; k < radix.size(); ++k)
+        std::copy(rv.begin() + rf[k], rv.begin() + rf[k + 1], h_values + h_rank_first[radix[k]]);
     return ADANA_OK;
 }
 

@@ -8,9 +8,9 @@ tensor, then the sorted values at indices ``unique(int32(1.1**k) - 1)``
 (clamped to n - 1) from the smallest end and from the largest end.
 
 Here the same indices are computed the same way on the host, and the values
-at those ranks come from the library's exact multi-rank radix select
-(``adana_order_stats``, adana_amd/csrc/adana_order_stats.hip): 4 to 8 passes
-over each tensor in HBM, nothing copied to the host but the selected values.
+at those ranks come from the library's exact multi-rank select
+(``adana_order_stats_sampled``, adana_amd/csrc/adana_order_sampled.h): two
+reads of each tensor in HBM, nothing copied to the host but the selected values.
 Results equal the reference's (float32 values; NaN sorts last as in
 np.sort).
 """
@@ -40,11 +40,11 @@ def order_stat_indices(n: int) -> np.ndarray:
 
 def _select(flat: Sequence[torch.Tensor], numel: np.ndarray, ranks: np.ndarray,
             rank_first: np.ndarray, compact: bool = True) -> np.ndarray:
-    """One adana_order_stats call: the values at ``ranks[rank_first[i]:
-    rank_first[i + 1]]`` of each contiguous float32 tensor ``flat[i]``,
-    concatenated.  ``compact``: give it the workspace with which its late
-    passes read only the values that can still match (about 1/8 of the
-    tensors' bytes more; same results)."""
+    """The values at ``ranks[rank_first[i]:rank_first[i + 1]]`` of each
+    contiguous float32 tensor ``flat[i]``, concatenated.  ``compact``: the
+    sampled select, which reads the tensors twice and keeps the values that
+    can still match (workspace of about 1/8 of the tensors' bytes);
+    otherwise the radix select without such a buffer (same results)."""
     dev = flat[0].device
     for f in flat:
         if f.device.type != "cuda" or f.dtype != torch.float32:
@@ -58,18 +58,19 @@ def _select(flat: Sequence[torch.Tensor], numel: np.ndarray, ranks: np.ndarray,
     ranks = ranks if total else np.zeros(1, np.int64)
     L = _lib.lib()
     if compact:
-        nbytes = int(L.adana_order_stats_workspace_compact(ctypes.c_void_p(numel.ctypes.data),
-                                                             ctypes.c_void_p(rank_first.ctypes.data), n))
+        select, name = L.adana_order_stats_sampled, "adana_order_stats_sampled"
+        nbytes = int(L.adana_order_stats_sampled_workspace(ctypes.c_void_p(numel.ctypes.data),
+                                                           ctypes.c_void_p(rank_first.ctypes.data), n))
     else:
+        select, name = L.adana_order_stats, "adana_order_stats"
         nbytes = int(L.adana_order_stats_workspace(n, total))
     ws = torch.empty(max(nbytes, 1), dtype=torch.uint8, device=dev)
     with torch.cuda.device(dev):
         stream = torch.cuda.current_stream(dev).cuda_stream
-        _lib.check(L.adana_order_stats(ctypes.c_void_p(ptrs.ctypes.data), ctypes.c_void_p(numel.ctypes.data),
-                                       n, ctypes.c_void_p(ranks.ctypes.data),
-                                       ctypes.c_void_p(rank_first.ctypes.data),
-                                       ctypes.c_void_p(values.ctypes.data), ctypes.c_void_p(ws.data_ptr()),
-                                       ws.numel(), ctypes.c_void_p(stream)), "adana_order_stats")
+        _lib.check(select(ctypes.c_void_p(ptrs.ctypes.data), ctypes.c_void_p(numel.ctypes.data), n,
+                          ctypes.c_void_p(ranks.ctypes.data), ctypes.c_void_p(rank_first.ctypes.data),
+                          ctypes.c_void_p(values.ctypes.data), ctypes.c_void_p(ws.data_ptr()), ws.numel(),
+                          ctypes.c_void_p(stream)), name)
     return values
 
 
