@@ -59,10 +59,16 @@ class GradPlan:
         self.chunk_first = None
         self.workspace = None
 
-    def prepare(self, grads: List[torch.Tensor]) -> None:
+    def prepare(self, grads: List[torch.Tensor], numels: Optional[np.ndarray] = None,
+                ptrs: Optional[np.ndarray] = None) -> None:
+        """Lay out (if the sizes changed) and point the plan at ``grads``;
+        ``numels`` and ``ptrs``: their numel()s and data pointers, where the
+        caller has them."""
         n = len(grads)
-        numels = np.fromiter((g.numel() for g in grads), dtype=np.int64, count=n)
-        ptrs = np.frombuffer(_hoststep.data_ptrs(grads), dtype=np.uint64)
+        if numels is None:
+            numels = np.fromiter((g.numel() for g in grads), dtype=np.int64, count=n)
+        if ptrs is None:
+            ptrs = np.frombuffer(_hoststep.data_ptrs(grads), dtype=np.uint64)
         relayout = self.numels is None or not np.array_equal(numels, self.numels)
         self.grads = grads
         with torch.cuda.device(self.device):
@@ -124,8 +130,8 @@ _PLANS: "OrderedDict[tuple, GradPlan]" = OrderedDict()
 _MAX_PLANS = 8
 
 
-def _shared_plan(device, bf16: bool, grads) -> GradPlan:
-    key = (device, bf16, len(grads), hash(tuple(g.numel() for g in grads)))
+def _shared_plan(device, bf16: bool, numels: np.ndarray) -> GradPlan:
+    key = (device, bf16, numels.size, hash(numels.tobytes()))
     plan = _PLANS.get(key)
     if plan is None:
         plan = _PLANS[key] = GradPlan(device, bf16)
@@ -173,15 +179,26 @@ def clip_grad_norm_(parameters: Union[torch.Tensor, Iterable[torch.Tensor]], max
         raise NotImplementedError(f"clip_grad_norm_: norm_type {norm_type} (only 2.0 is implemented)")
     if optimizer is not None:
         optimizer.flush_clip()          # a pending scale applies before this norm is taken
-    grads = [p.grad for p in parameters if p.grad is not None]
-    if not grads:
-        return torch.tensor(0.0)
-    device, bf16 = _validate(grads)
+    found = _hoststep.clip_scan(parameters)
+    if found is not None:
+        grads, numels, ptrs, index, bf16 = found
+        if not grads:
+            return torch.tensor(0.0)
+        device = torch.device("cuda", index)
+        numels = np.frombuffer(numels, dtype=np.int64)
+        ptrs = np.frombuffer(ptrs, dtype=np.uint64)
+    else:
+        grads = [p.grad for p in parameters if p.grad is not None]
+        if not grads:
+            return torch.tensor(0.0)
+        device, bf16 = _validate(grads)
+        numels = np.fromiter((g.numel() for g in grads), dtype=np.int64, count=len(grads))
+        ptrs = None
     if optimizer is not None:
         plan = optimizer._clip_plan(device, bf16)
     else:
-        plan = _shared_plan(device, bf16, grads)
-    plan.prepare(grads)
+        plan = _shared_plan(device, bf16, numels)
+    plan.prepare(grads, numels, ptrs)
     clip = plan.clip_norm(max_norm)
     total = clip[0]
     if bf16:

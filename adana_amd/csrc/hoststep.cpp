@@ -26,6 +26,7 @@
  * state dicts, refreshed in place by each step, with any the caller still
  * refers to moved aside first.
  */
+#define PY_SSIZE_T_CLEAN
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/csrc/autograd/variable.h>
 #include <ATen/ops/from_blob.h>
@@ -446,6 +447,95 @@ PyObject *grads_match(PyObject *, PyObject *args) {
         PyErr_SetString(PyExc_RuntimeError, e.what());
         return nullptr;
     }
+    Py_RETURN_TRUE;
+}
+
+/* clip_scan(params) -> (grads, numels, ptrs, device_index, bf16) or None
+ *
+ * The gradients of the parameters that have one, their numel()s and data
+ * pointers as native int64 / uint64 bytes, for gradient clipping: one pass in
+ * place of a Python walk (10,000 gradients: 14 ms there).  None unless every
+ * parameter and gradient is exactly a torch tensor and the gradients are
+ * strided, float32 or bfloat16, of one dtype on one GPU, and fill their memory
+ * without gaps or overlap; the caller then checks them one by one (and raises
+ * the precise error). */
+PyObject *clip_scan(PyObject *, PyObject *args) {
+    PyObject *params;
+    if (!PyArg_ParseTuple(args, "O!", &PyList_Type, &params)) return nullptr;
+    const size_t n = static_cast<size_t>(PyList_GET_SIZE(params));
+    for (size_t i = 0; i < n; ++i)
+        if (!THPVariable_CheckExact(PyList_GET_ITEM(params, i))) Py_RETURN_NONE;
+    PyObject *grads = PyList_New(0);
+    if (!grads) return nullptr;
+    std::vector<int64_t> numel;
+    std::vector<uint64_t> ptr;
+    c10::ScalarType type = c10::ScalarType::Undefined;
+    c10::Device device(c10::DeviceType::CPU);
+    bool fits = true;
+    try {
+        numel.reserve(n);
+        ptr.reserve(n);
+        ScanPrefetch pf{reinterpret_cast<PyListObject *>(params)->ob_item, n};
+        for (size_t i = 0; i < n && fits; ++i) {
+            pf.ahead(i);
+            const at::Tensor &g = impl_of(PyList_GET_ITEM(params, static_cast<Py_ssize_t>(i)))->grad();
+            if (!g.defined()) continue;
+            if (numel.empty()) {
+                type = g.scalar_type();
+                device = g.device();
+            }
+            fits = g.layout() == c10::kStrided && device.is_cuda() && g.device() == device && g.scalar_type() == type &&
+                   (type == c10::ScalarType::Float || type == c10::ScalarType::BFloat16) &&
+                   g.is_non_overlapping_and_dense();
+            if (!fits) break;
+            PyObject *o = THPVariable_Wrap(g);
+            if (!o) {
+                Py_DECREF(grads);
+                return nullptr;
+            }
+            fits = THPVariable_CheckExact(o);
+            const int rc = PyList_Append(grads, o);
+            Py_DECREF(o);
+            if (rc) {
+                Py_DECREF(grads);
+                return nullptr;
+            }
+            numel.push_back(g.numel());
+            ptr.push_back(reinterpret_cast<uint64_t>(g.data_ptr()));
+        }
+    } catch (const std::exception &e) {
+        Py_DECREF(grads);
+        PyErr_SetString(PyExc_RuntimeError, e.what());
+        return nullptr;
+    }
+    if (!fits) {
+        Py_DECREF(grads);
+        Py_RETURN_NONE;
+    }
+    const Py_ssize_t bytes = static_cast<Py_ssize_t>(8 * numel.size());
+    return Py_BuildValue("(Ny#y#iO)", grads, reinterpret_cast<const char *>(numel.data()), bytes,
+                         reinterpret_cast<const char *>(ptr.data()), bytes, static_cast<int>(device.index()),
+                         type == c10::ScalarType::BFloat16 ? Py_True : Py_False);
+}
+
+/* grads_are(params, grads) -> bool: grads is, tensor for tensor, the list of
+ * the gradients of the parameters that have one.  False also for objects that
+ * are not exactly torch tensors. */
+PyObject *grads_are(PyObject *, PyObject *args) {
+    PyObject *params, *grads;
+    if (!PyArg_ParseTuple(args, "O!O!", &PyList_Type, &params, &PyList_Type, &grads)) return nullptr;
+    const Py_ssize_t n = PyList_GET_SIZE(params), m = PyList_GET_SIZE(grads);
+    Py_ssize_t k = 0;
+    for (Py_ssize_t i = 0; i < n; ++i) {
+        PyObject *p = PyList_GET_ITEM(params, i);
+        if (!THPVariable_CheckExact(p)) Py_RETURN_FALSE;
+        const at::Tensor &g = impl_of(p)->grad();
+        if (!g.defined()) continue;
+        if (k == m) Py_RETURN_FALSE;
+        PyObject *o = PyList_GET_ITEM(grads, k++);
+        if (!THPVariable_Check(o) || impl_of(o) != g.unsafeGetTensorImpl()) Py_RETURN_FALSE;
+    }
+    if (k != m) Py_RETURN_FALSE;
     Py_RETURN_TRUE;
 }
 
@@ -1333,6 +1423,11 @@ PyMethodDef methods[] = {
     {"grads_scan", grads_scan, METH_VARARGS,
      "grads_scan(params, bf16) -> (grads, absent, grad_ptrs, param_ptrs, match): grads_of, data_ptrs of the "
      "gradients and of the parameters, and grads_match, in one pass"},
+    {"clip_scan", clip_scan, METH_VARARGS,
+     "clip_scan(params) -> (grads, numels, ptrs, device_index, bf16), or None unless every gradient is a dense "
+     "float32 (or every one bfloat16) tensor on one GPU"},
+    {"grads_are", grads_are, METH_VARARGS,
+     "grads_are(params, grads) -> bool: grads is the list of the parameters' gradients (those that have one)"},
     {"advance_if_same", advance_if_same, METH_VARARGS,
      "advance_if_same(params, grads, states[, param_ptrs[, grad_ptrs]]) -> bool: if params[i].grad is "
      "grads[i] for all i (and params[i] / grads[i] still have the data pointers given as native uint64 bytes), "

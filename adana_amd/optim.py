@@ -386,6 +386,9 @@ class _DanaFamily(Optimizer):
         """Defer clip scaling to the next step() if ``grads`` are exactly the
         gradients that step will consume; False leaves the scaling to the caller."""
         params, _ = self._flat_params()
+        if _hoststep.grads_are(params, grads):       # the optimizer's own clip call: in its order
+            self._pending_clip = (grads, plan, clip, bool(write_back))
+            return True
         own = [g for g in map(_GRAD, params) if g is not None]
         if len(own) != len(grads):
             return False
