@@ -852,6 +852,15 @@ __device__ __forceinline__ void store_grad1(const void *g, int64_t off, float x)
 //             every op rounded to bfloat16 (update_n16).
 enum ParamMode { PM_F32 = 0, PM_MASTER = 1, PM_BF16 = 2 };
 
+// Whether the scaled gradients are stored.  A coefficient of exactly 1 (the norm
+// is within bounds, so every gradient is finite) leaves each as it is: nothing to
+// write back.  On 67 tensors of 51M float32 values the step then takes 299 us
+// instead of 346.  (Compared as an integer in an SGPR: as a float comparison the
+// same test made the unscaled step of that list 1.5% slower.)
+__device__ __forceinline__ bool writes_back(const ScalarPack &pack, float gs) {
+    return pack.write_grad && __builtin_amdgcn_readfirstlane(__float_as_int(gs)) != 0x3f800000;
+}
+
 // One thread's elements of tensor d from element `off` on (`left` of them
 // remain in the tensor; VEC at most are processed), with their diagnostics
 // terms added to acc.  UNIFORM: every thread of the workgroup works on this
@@ -889,7 +898,7 @@ __device__ __forceinline__ void thread_elems(const adana_tensor_desc &d, const v
             if (scaled) {
 #pragma unroll
                 for (int k = 0; k < VEC; ++k) G[k] = scale_grad<true>(G[k], gs);
-                if (pack.write_grad) store_grad_n<true, VEC>(grad, off, G);
+                if (writes_back(pack, gs)) store_grad_n<true, VEC>(grad, off, G);
             }
             update_n<STAR, POWK, NUM, VEC>(P, G, M, V, T, sc, tab, acc);
             st_bf16_n<VEC>(pp, P);
@@ -902,7 +911,7 @@ __device__ __forceinline__ void thread_elems(const adana_tensor_desc &d, const v
                 float g = load_grad1<true>(grad, off + e);
                 if (scaled) {
                     g = scale_grad<true>(g, gs);
-                    if (pack.write_grad) store_grad1<true>(grad, off + e, g);
+                    if (writes_back(pack, gs)) store_grad1<true>(grad, off + e, g);
                 }
                 const float o = update_elem<STAR, POWK, NUM>(bf16_to_f32(pp[e]), g, mm, vv, tt, sc, tab, acc);
                 pp[e] = f32_to_bf16(o);
@@ -934,7 +943,7 @@ __device__ __forceinline__ void thread_elems(const adana_tensor_desc &d, const v
             if (scaled) {
 #pragma unroll
                 for (int k = 0; k < VEC; ++k) G[k] = scale_grad<true>(G[k], gs);
-                if (pack.write_grad) store_grad_n<true, VEC>(grad, off, G);
+                if (writes_back(pack, gs)) store_grad_n<true, VEC>(grad, off, G);
             }
             update_n16<STAR, POWK, VEC, NUM == NUM_FOREACH_EAGER16>(P, G, M, V, T, sc, q, tab, acc);
             st_bf16_n<VEC>(pp, P);
@@ -948,7 +957,7 @@ __device__ __forceinline__ void thread_elems(const adana_tensor_desc &d, const v
                 float G[1] = {load_grad1<true>(grad, off + e)};
                 if (scaled) {
                     G[0] = scale_grad<true>(G[0], gs);
-                    if (pack.write_grad) store_grad1<true>(grad, off + e, G[0]);
+                    if (writes_back(pack, gs)) store_grad1<true>(grad, off + e, G[0]);
                 }
                 update_n16<STAR, POWK, 1, NUM == NUM_FOREACH_EAGER16>(P, G, M, V, T, sc, q, tab, acc);
                 pp[e] = f32_to_bf16(P[0]);
@@ -978,7 +987,7 @@ __device__ __forceinline__ void thread_elems(const adana_tensor_desc &d, const v
         if (scaled) {
 #pragma unroll
             for (int k = 0; k < VEC; ++k) G[k] = scale_grad<GBF16>(G[k], gs);
-            if (pack.write_grad) store_grad_n<GBF16, VEC>(grad, off, G);
+            if (writes_back(pack, gs)) store_grad_n<GBF16, VEC>(grad, off, G);
         }
         update_n<STAR, POWK, NUM, VEC>(P, G, M, V, T, sc, tab, acc);
         if constexpr (UNIFORM && VEC == 4) {
@@ -1001,7 +1010,7 @@ __device__ __forceinline__ void thread_elems(const adana_tensor_desc &d, const v
             float g = load_grad1<GBF16>(grad, off + e);
             if (scaled) {
                 g = scale_grad<GBF16>(g, gs);
-                if (pack.write_grad) store_grad1<GBF16>(grad, off + e, g);
+                if (writes_back(pack, gs)) store_grad1<GBF16>(grad, off + e, g);
             }
             const float o = update_elem<STAR, POWK, NUM>(pp[e], g, mm, vv, tt, sc, tab, acc);
             pp[e] = o;
@@ -1060,7 +1069,8 @@ __device__ __forceinline__ bool thread_groups_uniform(const adana_tensor_desc &d
             for (int k = 0; k < GROUPS; ++k) {
 #pragma unroll
                 for (int e = 0; e < VEC; ++e) G[k][e] = scale_grad<GBF16>(G[k][e], gs);
-                if (pack.write_grad) store_grad_n<GBF16, VEC>(grad, off + static_cast<int64_t>(k) * span, G[k]);
+                if (writes_back(pack, gs))
+                    store_grad_n<GBF16, VEC>(grad, off + static_cast<int64_t>(k) * span, G[k]);
             }
         }
 #pragma unroll
@@ -1450,32 +1460,41 @@ __global__ __launch_bounds__(kBlock) void combine_kernel(const adana_tensor_desc
 // Sum of squares per (chunk, tensor) segment in binary64 (each square of a
 // binary32 value is exact in binary64), written to partials[chunk + tensor].x.
 // One workgroup covers kSumsqChunks consecutive chunks.  When they all lie in
-// one tensor with aligned vectors (every chunk of a large tensor but its
-// ends), each thread issues its kSumsqChunks 16-byte loads at once and the
-// per-chunk sums are reduced together; otherwise the chunks are walked one by
-// one, segment by segment.  Either way each chunk's partial is the same
-// fixed-order sum of its own elements.
-constexpr int kSumsqChunks = 4;
+// one tensor and start on a 16-byte boundary (every chunk of a large tensor but
+// its ends), each thread issues its 16-byte loads at once, the workgroup makes
+// one sum of all its chunks and stores it in the first one's slot (zero in the
+// others'); otherwise each wave walks a chunk, segment by segment.  Either way
+// the sums are in a fixed order.  Bound by the reads: 1.31G bfloat16 values 406
+// us, 6.5 TB/s (8-byte loads and four reductions per workgroup took 701 us, 3.7
+// TB/s); 51M float32 values in 67 tensors 36.5 us (42.6); 95M in 10,000 tensors,
+// where a workgroup walked its chunks one after another, 65 us (80).
+template <bool GBF16>
+constexpr int kSumsqChunks = GBF16 ? 8 : 4;
 
+// One wave: the chunk's segments, each lane four vectors of each.
 template <bool GBF16>
 __device__ __forceinline__ void sumsq_chunk(const adana_tensor_desc *__restrict__ desc,
                                               const void *const *__restrict__ gradp,
                                               const int64_t *__restrict__ vstart, int first, int32_t n,
-                                              int64_t chunk, double2 *__restrict__ partials, double (*red)[kWaves]) {
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+                                              int64_t chunk, double2 *__restrict__ partials) {
+    constexpr int kVecs = kChunk / (4 * 64);
+    const int lane = threadIdx.x & 63;
     const int64_t lo = chunk * kChunk, hi = lo + kChunk;
-    const int64_t mine = lo + 4 * tid;
     for (int i = first; i < n; ++i) {
         const int64_t vs = vstart[i];
         if (vs >= hi) break;
         const int64_t ve = vs + desc[i].numel;
         if (ve <= lo) continue;
         const void *grad = gradp[i];
+        const bool vec_ok = grad_vec_aligned<GBF16>(grad);
         double acc = 0.0;
-        if (mine >= vs && mine < ve) {
+#pragma unroll
+        for (int u = 0; u < kVecs; ++u) {
+            const int64_t mine = lo + 4 * (lane + 64 * u);
+            if (mine < vs || mine >= ve) continue;
             const int64_t off = mine - vs;
             const int cnt = (ve - mine) < 4 ? static_cast<int>(ve - mine) : 4;
-            if (cnt == 4 && grad_vec_aligned<GBF16>(grad)) {
+            if (cnt == 4 && vec_ok) {
                 float G[4];
                 load_grad_n<GBF16, 4>(grad, off, G);
 #pragma unroll
@@ -1489,10 +1508,37 @@ __device__ __forceinline__ void sumsq_chunk(const adana_tensor_desc *__restrict_
         }
 #pragma unroll
         for (int o = 32; o > 0; o >>= 1) acc += __shfl_xor(acc, o, 64);
-        if (lane == 0) red[0][wave] = acc;
-        __syncthreads();
-        if (tid == 0) partials[chunk + i] = make_double2(((red[0][0] + red[0][1]) + red[0][2]) + red[0][3], 0.0);
-        __syncthreads();
+        if (lane == 0) partials[chunk + i] = make_double2(acc, 0.0);
+    }
+}
+
+// 16 bytes of a gradient: 4 float32 or 8 bfloat16 values.
+template <bool GBF16>
+__device__ __forceinline__ void load_grad16(const void *g, int64_t off, float (&o)[GBF16 ? 8 : 4]) {
+    if constexpr (GBF16) {
+        typedef unsigned int H4 __attribute__((ext_vector_type(4)));
+        const H4 h = __builtin_nontemporal_load((const GLOBAL_AS H4 *)(static_cast<const unsigned short *>(g) + off));
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            o[2 * k] = __uint_as_float(h[k] << 16);
+            o[2 * k + 1] = __uint_as_float(h[k] & 0xffff0000u);
+        }
+    } else {
+        load_grad_n<false, 4>(g, off, o);
+    }
+}
+
+template <bool GBF16>
+__device__ __forceinline__ void store_grad16(const void *g, int64_t off, const float (&x)[GBF16 ? 8 : 4]) {
+    if constexpr (GBF16) {
+        typedef unsigned int H4 __attribute__((ext_vector_type(4)));
+        H4 h;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) h[k] = adana::bf16_pack2(x[2 * k], x[2 * k + 1]);
+        __builtin_nontemporal_store(
+            h, (GLOBAL_AS H4 *)(const_cast<unsigned short *>(static_cast<const unsigned short *>(g)) + off));
+    } else {
+        store_grad_n<false, 4>(g, off, x);
     }
 }
 
@@ -1503,8 +1549,10 @@ __global__ __launch_bounds__(kBlock) void grad_sumsq_kernel(const adana_tensor_d
                                                             const int32_t *__restrict__ chunk_first,
                                                             int32_t n, int64_t n_chunks,
                                                             double2 *__restrict__ partials) {
-    constexpr int K = kSumsqChunks;
-    __shared__ double red[K][kWaves];
+    constexpr int K = kSumsqChunks<GBF16>;
+    constexpr int kVals = GBF16 ? 8 : 4;                     // of a 16-byte load
+    constexpr int kLoads = K * kChunk / (kBlock * kVals);
+    __shared__ double red[kWaves];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int64_t c0 = static_cast<int64_t>(blockIdx.x) * K;
     const int64_t nc = (n_chunks - c0) < K ? n_chunks - c0 : K;
@@ -1512,44 +1560,61 @@ __global__ __launch_bounds__(kBlock) void grad_sumsq_kernel(const adana_tensor_d
     const int64_t vs = vstart[i0];
     const int64_t numel0 = desc[i0].numel;
     const void *g0 = gradp[i0];
-    if (nc == K && vs <= c0 * kChunk && vs + numel0 >= (c0 + K) * kChunk && grad_vec_aligned<GBF16>(g0)) {
-        const int64_t off0 = c0 * kChunk + 4 * tid - vs;
-        float G[K][4];
+    const int64_t seg0 = c0 * kChunk - vs;
+    const bool aligned = ((reinterpret_cast<uintptr_t>(g0) + static_cast<uint64_t>(seg0) * (GBF16 ? 2 : 4)) & 15u) == 0;
+    if (nc == K && seg0 >= 0 && vs + numel0 >= (c0 + K) * kChunk && aligned) {
+        float G[kLoads][kVals];
 #pragma unroll
-        for (int c = 0; c < K; ++c) load_grad_n<GBF16, 4>(g0, off0 + c * kChunk, G[c]);
-        double acc[K];
+        for (int u = 0; u < kLoads; ++u) load_grad16<GBF16>(g0, seg0 + (u * kBlock + tid) * kVals, G[u]);
+        double acc = 0.0;
 #pragma unroll
-        for (int c = 0; c < K; ++c) {
-            acc[c] = 0.0;
+        for (int u = 0; u < kLoads; ++u) {
 #pragma unroll
-            for (int k = 0; k < 4; ++k) acc[c] += static_cast<double>(G[c][k]) * static_cast<double>(G[c][k]);
+            for (int k = 0; k < kVals; ++k) {
+                const double g = G[u][k];
+                acc = __builtin_fma(g, g, acc);              // the square is exact: the same as a sum of squares
+            }
         }
 #pragma unroll
-        for (int o = 32; o > 0; o >>= 1) {
-#pragma unroll
-            for (int c = 0; c < K; ++c) acc[c] += __shfl_xor(acc[c], o, 64);
-        }
-        if (lane == 0) {
-#pragma unroll
-            for (int c = 0; c < K; ++c) red[c][wave] = acc[c];
-        }
+        for (int o = 32; o > 0; o >>= 1) acc += __shfl_xor(acc, o, 64);
+        if (lane == 0) red[wave] = acc;
         __syncthreads();
         if (tid < K)
-            partials[c0 + tid + i0] = make_double2(((red[tid][0] + red[tid][1]) + red[tid][2]) + red[tid][3], 0.0);
+            partials[c0 + tid + i0] =
+                make_double2(tid == 0 ? ((red[0] + red[1]) + red[2]) + red[3] : 0.0, 0.0);
         return;
     }
-    for (int c = 0; c < nc; ++c) sumsq_chunk<GBF16>(desc, gradp, vstart, chunk_first[c0 + c], n, c0 + c, partials, red);
+    for (int c = wave; c < nc; c += kWaves)
+        sumsq_chunk<GBF16>(desc, gradp, vstart, chunk_first[c0 + c], n, c0 + c, partials);
 }
 
-// Stage 1 of the norm combine: like the fold workgroups of combine_kernel, for one
-// binary64 sum.
+// Stage 1 of the norm combine, as combine_kernel's for one binary64 sum: the
+// first n_folds workgroups reduce a fold each; the others take four tensors of
+// at most ADANA_DIRECT_CHUNKS chunks each, one wave per tensor, and leave the
+// tensor's sum in its first slot's second half (zero for an empty tensor).
 __global__ __launch_bounds__(kBlock) void sumsq_fold_kernel(const adana_tensor_desc *__restrict__ desc,
                                                             const int64_t *__restrict__ vstart,
                                                             const int32_t *__restrict__ fold_first, int32_t n,
-                                                            const double2 *__restrict__ partials,
+                                                            int32_t n_folds, double2 *__restrict__ partials,
                                                             double *__restrict__ folds) {
     __shared__ double red[kWaves];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int64_t j = blockIdx.x;
+    if (j >= n_folds) {
+        const int i = static_cast<int>((j - n_folds) * kWaves + wave);
+        if (i >= n || fold_first[i + 1] > fold_first[i]) return;             // whole wave
+        const int64_t numel = desc[i].numel, b0 = vstart[i] / kChunk;
+        double s = 0.0;
+        if (numel > 0) {
+            const int64_t b1 = (vstart[i] + numel - 1) / kChunk;
+#pragma unroll 8
+            for (int64_t b = b0 + lane; b <= b1; b += 64) s += partials[b + i].x;
+        }
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+        if (lane == 0) partials[b0 + i].y = s;
+        return;
+    }
     int l = 0, r = n - 1;
     while (l < r) {
         const int mid = (l + r + 1) >> 1;
@@ -1566,7 +1631,6 @@ __global__ __launch_bounds__(kBlock) void sumsq_fold_kernel(const adana_tensor_d
         const int64_t b = lo + u * kBlock + threadIdx.x;
         if (b <= hi) s += partials[b + i].x;
     }
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
     if (lane == 0) red[wave] = s;
@@ -1583,9 +1647,16 @@ __global__ __launch_bounds__(kBlock) void sumsq_fold_kernel(const adana_tensor_d
 // Each op rounds to the gradient dtype (bfloat16 gradients give bfloat16
 // norms and coefficient).  clip[0] = total norm, clip[1] = coefficient.
 constexpr int kClipThreads = 1024;
-// One wave per tensor (tensors w, w + 16, ... for wave w) sums the tensor's
-// folds, or its chunk partials directly when it has no folds.
-template <bool GBF16>
+// SUMMED: sumsq_fold_kernel has run.  Each lane takes a tensor, 16 apart within a
+// wave, and sums its few folds; more than kLaneFolds folds (an embedding) are
+// summed by the whole wave.  (A wave per tensor, 16 tensors at a time, each behind
+// four dependent reads, took 863 us for a list of 10,000 tensors, now 22, and
+// 8.4 us for 67, now 4.2.)  Not SUMMED, for lists of up to kClipDirect tensors
+// without folds: a wave per tensor sums its chunk partials, which saves the
+// launch between.
+constexpr int kLaneFolds = 64;
+constexpr int kClipDirect = 32;
+template <bool GBF16, bool SUMMED>
 __global__ __launch_bounds__(kClipThreads) void clip_finalize_kernel(const adana_tensor_desc *__restrict__ desc,
                                                                      const int64_t *__restrict__ vstart,
                                                                      const int32_t *__restrict__ fold_first,
@@ -1596,24 +1667,57 @@ __global__ __launch_bounds__(kClipThreads) void clip_finalize_kernel(const adana
     constexpr int kClipWaves = kClipThreads / 64;
     __shared__ double red[kClipWaves];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    double tot = 0.0;                                    // lane 0: this wave's tensors, in order
-    for (int i = wave; i < n; i += kClipWaves) {
-        double s = 0.0;
-        const int64_t numel = desc[i].numel;
-        if (fold_first[i + 1] > fold_first[i]) {
-            for (int f = fold_first[i] + lane; f < fold_first[i + 1]; f += 64) s += folds[f];
-        } else if (numel > 0) {
-            const int64_t b0 = vstart[i] / kChunk, b1 = (vstart[i] + numel - 1) / kChunk;
+    auto norm_of = [](double s) {
+        const float nrm = static_cast<float>(sqrt(s));
+        return GBF16 ? bf16_round(nrm) : nrm;
+    };
+    double tot = 0.0;                                    // this lane's tensors, in order
+    if constexpr (SUMMED) {
+        for (int base = wave; base < n; base += kClipThreads) {
+            const int i = base + kClipWaves * lane;
+            const int f0 = i < n ? fold_first[i] : 0, f1 = i < n ? fold_first[i + 1] : 0;
+            double s = 0.0;
+            if (i < n && f0 == f1) s = partials[vstart[i] / kChunk + i].y;
+            if (f1 - f0 <= kLaneFolds) {
 #pragma unroll 8
-            for (int64_t b = b0 + lane; b <= b1; b += 64) s += partials[b + i].x;
+                for (int f = f0; f < f1; ++f) s += folds[f];
+            }
+            uint64_t folded = __ballot(f1 - f0 > kLaneFolds);
+            while (folded) {
+                const int l = __ffsll(static_cast<unsigned long long>(folded)) - 1;
+                folded &= folded - 1;
+                const int a = __shfl(f0, l, 64), b = __shfl(f1, l, 64);
+                double q = 0.0;
+#pragma unroll 4
+                for (int f = a + lane; f < b; f += 64) q += folds[f];
+#pragma unroll
+                for (int o = 32; o > 0; o >>= 1) q += __shfl_xor(q, o, 64);
+                if (lane == l) s = q;
+            }
+            if (i < n) {
+                const float nrm = norm_of(s);
+                if (norms) norms[i] = nrm;
+                tot += static_cast<double>(nrm) * static_cast<double>(nrm);
+            }
         }
 #pragma unroll
-        for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
-        float nrm = static_cast<float>(sqrt(s));
-        if (GBF16) nrm = bf16_round(nrm);
-        if (lane == 0) {
-            if (norms) norms[i] = nrm;
-            tot += static_cast<double>(nrm) * static_cast<double>(nrm);
+        for (int o = 32; o > 0; o >>= 1) tot += __shfl_xor(tot, o, 64);
+    } else {
+        for (int i = wave; i < n; i += kClipWaves) {
+            double s = 0.0;
+            const int64_t numel = desc[i].numel;
+            if (numel > 0) {
+                const int64_t b0 = vstart[i] / kChunk, b1 = (vstart[i] + numel - 1) / kChunk;
+#pragma unroll 8
+                for (int64_t b = b0 + lane; b <= b1; b += 64) s += partials[b + i].x;
+            }
+#pragma unroll
+            for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+            const float nrm = norm_of(s);
+            if (lane == 0) {
+                if (norms) norms[i] = nrm;
+                tot += static_cast<double>(nrm) * static_cast<double>(nrm);
+            }
         }
     }
     if (lane == 0) red[wave] = tot;
@@ -1636,34 +1740,66 @@ __global__ __launch_bounds__(kClipThreads) void clip_finalize_kernel(const adana
 }
 
 // In-place g *= coef over a gradient list (clip_grad_norm_ without a fused
-// optimizer step).
+// optimizer step).  A workgroup covers as many chunks as in grad_sumsq_kernel,
+// with all its 16-byte loads in flight when they lie in one tensor.  A
+// coefficient of exactly 1 (the norm is within bounds, so every gradient is
+// finite) leaves each value as it is: nothing is read or written.  1.31G bfloat16
+// values at a coefficient of 1: 35 us, the launch of the workgroups (one chunk
+// per workgroup with 8-byte loads, and no such test, took 1,156 us).
 template <bool GBF16>
 __global__ __launch_bounds__(kBlock) void grad_scale_kernel(const adana_tensor_desc *__restrict__ desc,
                                                             const void *const *__restrict__ gradp,
                                                             const int64_t *__restrict__ vstart,
                                                             const int32_t *__restrict__ chunk_first,
-                                                            int32_t n, const float *__restrict__ scale) {
-    const int64_t chunk = blockIdx.x;
-    const int64_t lo = chunk * kChunk, hi = lo + kChunk;
-    const int64_t mine = lo + 4 * threadIdx.x;
+                                                            int32_t n, int64_t n_chunks,
+                                                            const float *__restrict__ scale) {
+    constexpr int K = kSumsqChunks<GBF16>;
+    constexpr int kVals = GBF16 ? 8 : 4;
+    constexpr int kLoads = K * kChunk / (kBlock * kVals);
+    const int tid = threadIdx.x;
+    const int64_t c0 = static_cast<int64_t>(blockIdx.x) * K;
     const float s = *scale;
-    for (int i = chunk_first[chunk]; i < n; ++i) {
-        const int64_t vs = vstart[i];
-        if (vs >= hi) break;
-        const int64_t ve = vs + desc[i].numel;
-        if (ve <= lo || mine < vs || mine >= ve) continue;
-        const void *grad = gradp[i];
-        const int64_t off = mine - vs;
-        const int cnt = (ve - mine) < 4 ? static_cast<int>(ve - mine) : 4;
-        if (cnt == 4 && grad_vec_aligned<GBF16>(grad)) {
-            float G[4];
-            load_grad_n<GBF16, 4>(grad, off, G);
+    const int i0 = chunk_first[c0];
+    const int64_t vs0 = vstart[i0];
+    const int64_t numel0 = desc[i0].numel;
+    const void *g0 = gradp[i0];
+    if (s == 1.0f) return;
+    const int64_t nc = (n_chunks - c0) < K ? n_chunks - c0 : K;
+    const int64_t seg0 = c0 * kChunk - vs0;
+    const bool aligned = ((reinterpret_cast<uintptr_t>(g0) + static_cast<uint64_t>(seg0) * (GBF16 ? 2 : 4)) & 15u) == 0;
+    if (nc == K && seg0 >= 0 && vs0 + numel0 >= (c0 + K) * kChunk && aligned) {
+        float G[kLoads][kVals];
 #pragma unroll
-            for (int k = 0; k < 4; ++k) G[k] = scale_grad<GBF16>(G[k], s);
-            store_grad_n<GBF16, 4>(grad, off, G);
-        } else {
-            for (int e = 0; e < cnt; ++e)
-                store_grad1<GBF16>(grad, off + e, scale_grad<GBF16>(load_grad1<GBF16>(grad, off + e), s));
+        for (int u = 0; u < kLoads; ++u) load_grad16<GBF16>(g0, seg0 + (u * kBlock + tid) * kVals, G[u]);
+#pragma unroll
+        for (int u = 0; u < kLoads; ++u) {
+#pragma unroll
+            for (int k = 0; k < kVals; ++k) G[u][k] = scale_grad<GBF16>(G[u][k], s);
+            store_grad16<GBF16>(g0, seg0 + (u * kBlock + tid) * kVals, G[u]);
+        }
+        return;
+    }
+    for (int c = 0; c < nc; ++c) {
+        const int64_t lo = (c0 + c) * kChunk, hi = lo + kChunk;
+        const int64_t mine = lo + 4 * tid;
+        for (int i = chunk_first[c0 + c]; i < n; ++i) {
+            const int64_t vs = vstart[i];
+            if (vs >= hi) break;
+            const int64_t ve = vs + desc[i].numel;
+            if (ve <= lo || mine < vs || mine >= ve) continue;
+            const void *grad = gradp[i];
+            const int64_t off = mine - vs;
+            const int cnt = (ve - mine) < 4 ? static_cast<int>(ve - mine) : 4;
+            if (cnt == 4 && grad_vec_aligned<GBF16>(grad)) {
+                float G[4];
+                load_grad_n<GBF16, 4>(grad, off, G);
+#pragma unroll
+                for (int k = 0; k < 4; ++k) G[k] = scale_grad<GBF16>(G[k], s);
+                store_grad_n<GBF16, 4>(grad, off, G);
+            } else {
+                for (int e = 0; e < cnt; ++e)
+                    store_grad1<GBF16>(grad, off + e, scale_grad<GBF16>(load_grad1<GBF16>(grad, off + e), s));
+            }
         }
     }
 }
@@ -2356,24 +2492,30 @@ int adana_grad_clip_norm(const adana_plan *plan, uint32_t grad_flags, double max
     double *folds = reinterpret_cast<double *>(static_cast<char *>(d_workspace) + folds_offset(pl));
     const int32_t n = pl.n_tensors;
     if (pl.n_chunks > 0) {
-        const dim3 grid(static_cast<unsigned>((pl.n_chunks + kSumsqChunks - 1) / kSumsqChunks));
-        if (gb) hipLaunchKernelGGL(grad_sumsq_kernel<true>, grid, dim3(kBlock), 0, st, pl.desc, pl.grad,
-                                   pl.vstart, pl.chunk_first, n, pl.n_chunks, partials);
-        else hipLaunchKernelGGL(grad_sumsq_kernel<false>, grid, dim3(kBlock), 0, st, pl.desc, pl.grad,
-                                pl.vstart, pl.chunk_first, n, pl.n_chunks, partials);
+        constexpr int64_t k32 = kSumsqChunks<false>, k16 = kSumsqChunks<true>;
+        if (gb) hipLaunchKernelGGL(grad_sumsq_kernel<true>, dim3(static_cast<unsigned>((pl.n_chunks + k16 - 1) / k16)),
+                                   dim3(kBlock), 0, st, pl.desc, pl.grad, pl.vstart, pl.chunk_first, n, pl.n_chunks,
+                                   partials);
+        else hipLaunchKernelGGL(grad_sumsq_kernel<false>, dim3(static_cast<unsigned>((pl.n_chunks + k32 - 1) / k32)),
+                                dim3(kBlock), 0, st, pl.desc, pl.grad, pl.vstart, pl.chunk_first, n, pl.n_chunks,
+                                partials);
         if (int rc = launch_status(fn, "sum of squares")) return rc;
     }
-    if (pl.n_folds > 0) {
-        hipLaunchKernelGGL(sumsq_fold_kernel, dim3(static_cast<unsigned>(pl.n_folds)), dim3(kBlock), 0, st,
-                           pl.desc, pl.vstart, pl.fold_first, n, partials, folds);
+    const bool summed = pl.n_folds > 0 || n > kClipDirect;
+    if (summed) {
+        const int64_t tensor_wgs = (static_cast<int64_t>(n) + kWaves - 1) / kWaves;
+        hipLaunchKernelGGL(sumsq_fold_kernel, dim3(static_cast<unsigned>(pl.n_folds + tensor_wgs)), dim3(kBlock), 0, st,
+                           pl.desc, pl.vstart, pl.fold_first, n, static_cast<int32_t>(pl.n_folds), partials, folds);
         if (int rc = launch_status(fn, "fold")) return rc;
     }
     // torch casts the Python float max_norm to the coefficient's binary32 opmath
     const float mn = static_cast<float>(max_norm);
-    if (gb) hipLaunchKernelGGL(clip_finalize_kernel<true>, dim3(1), dim3(kClipThreads), 0, st, pl.desc, pl.vstart,
-                               pl.fold_first, n, partials, folds, mn, d_norms, d_clip);
-    else hipLaunchKernelGGL(clip_finalize_kernel<false>, dim3(1), dim3(kClipThreads), 0, st, pl.desc, pl.vstart,
-                            pl.fold_first, n, partials, folds, mn, d_norms, d_clip);
+#define ADANA_FINALIZE(G, S) \
+    hipLaunchKernelGGL((clip_finalize_kernel<G, S>), dim3(1), dim3(kClipThreads), 0, st, pl.desc, pl.vstart, \
+                       pl.fold_first, n, partials, folds, mn, d_norms, d_clip)
+    if (gb) { if (summed) ADANA_FINALIZE(true, true); else ADANA_FINALIZE(true, false); }
+    else    { if (summed) ADANA_FINALIZE(false, true); else ADANA_FINALIZE(false, false); }
+#undef ADANA_FINALIZE
     return launch_status(fn, "finalize");
 }
 
@@ -2386,13 +2528,14 @@ int adana_grad_scale(const adana_plan *plan, uint32_t grad_flags, const float *d
     if (!d_scale) return adana_set_error(ADANA_E_INVALID, "%s: null scale", fn);
     if (pl.n_tensors == 0 || pl.n_chunks == 0) return ADANA_OK;
     hipStream_t st = static_cast<hipStream_t>(stream);
-    const dim3 grid(static_cast<unsigned>(pl.n_chunks));
+    const int64_t k = grad_flags & ADANA_GRAD_BF16 ? kSumsqChunks<true> : kSumsqChunks<false>;
+    const dim3 grid(static_cast<unsigned>((pl.n_chunks + k - 1) / k));
     if (grad_flags & ADANA_GRAD_BF16)
         hipLaunchKernelGGL(grad_scale_kernel<true>, grid, dim3(kBlock), 0, st, pl.desc, pl.grad, pl.vstart,
-                           pl.chunk_first, pl.n_tensors, d_scale);
+                           pl.chunk_first, pl.n_tensors, pl.n_chunks, d_scale);
     else
         hipLaunchKernelGGL(grad_scale_kernel<false>, grid, dim3(kBlock), 0, st, pl.desc, pl.grad, pl.vstart,
-                           pl.chunk_first, pl.n_tensors, d_scale);
+                           pl.chunk_first, pl.n_tensors, pl.n_chunks, d_scale);
     return launch_status(fn, "scale");
 }
 

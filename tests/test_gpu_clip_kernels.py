@@ -1,0 +1,55 @@
+"""The norm, combine and scaling kernels of clip_grad_norm_ at the sizes where
+they change path: whole workgroups of 16-byte loads or segment by segment,
+tensors with and without folds (and more than 64 folds), lists short enough to
+be combined without the fold launch, empty tensors; norms that bind and that do
+not."""
+import numpy as np
+import pytest
+import torch
+
+import adana_amd
+
+pytestmark = [pytest.mark.gpu,
+              pytest.mark.skipif(not torch.cuda.is_available(), reason="needs a ROCm GPU")]
+
+DEV = "cuda:0"
+LISTS = {
+    "one value": [(1, 0)],
+    "workgroup edges": [(n, 0) for n in (4095, 4096, 4097, 8191, 8192, 8193, 16384 + 1024)],
+    "misaligned": [(20_000, k) for k in range(1, 9)],
+    "folds": [(512 * 1024, 0), (512 * 1024 + 1, 0), (3_000_001, 0), (700_000, 3), (5, 0)],
+    "many folds": [(64 * 512 * 1024 + 7, 0), (1000, 0)],
+    "32 small": [(1 + 37 * i, 0) for i in range(32)],
+    "33 small": [(1 + 37 * i, 0) for i in range(33)],
+    "2,100 with empty ones": [((i * 7919) % 3000 if i % 5 else 0, 0) for i in range(2100)],
+}
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("name", LISTS)
+def test_norm_and_scaling(name, dtype):
+    print(f"case: clip kernels, {name}, {dtype}", flush=True)
+    g = torch.Generator(device=DEV)
+    g.manual_seed(len(name))
+    params = []
+    for n, off in LISTS[name]:
+        p = torch.nn.Parameter(torch.zeros(n, dtype=dtype, device=DEV))
+        p.grad = torch.randn(n + off, device=DEV, generator=g).to(dtype)[off:]
+        params.append(p)
+    before = [p.grad.clone() for p in params]
+    norms = torch.stack([b.double().square().sum().sqrt() for b in before]).float()
+    want = float(norms.double().square().sum().sqrt())
+    if dtype == torch.bfloat16:
+        want = float(norms.to(dtype).double().square().sum().sqrt())
+    # binary32 norms of binary64 sums and one more rounding; bfloat16 norms may
+    # round to the neighbour, half a unit of 8 bits each way
+    rel = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -22
+    total = adana_amd.clip_grad_norm_(params, 10.0 * want)            # does not bind
+    assert abs(float(total) - want) <= rel * want
+    assert all(torch.equal(p.grad, b) for p, b in zip(params, before))
+    total = adana_amd.clip_grad_norm_(params, 0.25 * want)
+    t = total.to(dtype)
+    coef = torch.clamp(0.25 * want / (t + 1e-6), max=1.0)             # torch's order and dtype
+    assert float(coef) < 0.3
+    for p, b in zip(params, before):
+        assert torch.equal(p.grad, b * coef)
