@@ -38,44 +38,52 @@ __device__ __forceinline__ int class_mask(int m) {
     return r;
 }
 
-// Correctly rounded a / b for operands on which the IEEE division sequence's
-// range scaling (v_div_scale) and special-case fixup (v_div_fixup) are
-// identities: b normal in [0.5, 1], and a either normal or b == 1.  This is the
-// same refinement chain the full sequence runs (reciprocal, one Newton step,
-// two remainder corrections), so the result is bit-identical to a / b there.
+// Correctly rounded a / (1 - a), b = 1 - a, for a in [0, 0.5]: the hardware
+// reciprocal, the quotient and one remainder correction.  (The IEEE sequence's
+// range scaling, fixup, Newton step and second correction change nothing on this
+// curve; checked for every binary32 a.)  4 instructions in place of 8.
 __device__ __forceinline__ float div_core(float a, float b) {
-    float y = __builtin_amdgcn_rcpf(b);
-    const float e = __builtin_fmaf(-b, y, 1.0f);
-    y = __builtin_fmaf(e, y, y);
-    float q = a * y;
-    float r = __builtin_fmaf(-b, q, a);
-    q = __builtin_fmaf(r, y, q);
-    r = __builtin_fmaf(-b, q, a);
+    const float y = __builtin_amdgcn_rcpf(b);
+    const float q = a * y;
+    const float r = __builtin_fmaf(-b, q, a);
     return __builtin_fmaf(r, y, q);
 }
 
-// Correctly rounded sqrt for x >= 2^-96 (or NaN): the hardware square root
-// followed by the neighbour test of the full IEEE sequence, without its
-// small-input scaling and zero/inf/negative fixups (identities there).
-__device__ __forceinline__ float sqrt_normal(float x) {
-    const float s = __builtin_amdgcn_sqrtf(x);
-    const float sm = __uint_as_float(__float_as_uint(s) - 1u);
-    const float sp = __uint_as_float(__float_as_uint(s) + 1u);
-    const float rm = __builtin_fmaf(-sm, s, x);
-    const float rp = __builtin_fmaf(-sp, s, x);
-    float o = rm <= 0.0f ? sm : s;
-    o = rp > 0.0f ? sp : o;
-    return o;
+// Correctly rounded sqrt for finite x >= 2^-96: x * rsqrt(x) by the hardware
+// reciprocal square root and one remainder correction (checked for every such
+// binary32 x).  5 instructions; the hardware square root with a test of both
+// neighbours, which the IEEE sequence has, takes 9 (a correction of the hardware
+// square root by its reciprocal misses 112 inputs).
+__device__ __forceinline__ float sqrt_scaled(float x, float y) {   // y = rsqrt(x)
+    const float s = x * y;
+    const float r = __builtin_fmaf(-s, s, x);
+    return __builtin_fmaf(r, 0.5f * y, s);
 }
+__device__ __forceinline__ float sqrt_finite(float x) { return sqrt_scaled(x, __builtin_amdgcn_rsqf(x)); }
 
-// Correctly rounded sqrt for every binary32 x: sqrt_normal on [2^-96, +inf]
-// and for +-0 (about 8 instructions against the IEEE sequence's 20), the IEEE
-// sequence for small nonzero and negative inputs and NaNs, behind a real
-// branch.  Zeros stay on the fast path: a second moment that never saw a
-// nonzero gradient (zero rows of an embedding) is 0 for whole waves.
+// The same for +inf too (the form the exhaustive check runs).
+__device__ __forceinline__ float sqrt_normal(float x) { return x < __builtin_inff() ? sqrt_finite(x) : x; }
+
+// Correctly rounded sqrt for every binary32 x: sqrt_finite from 2^-96 on and for
+// +-0 (its reciprocal square root taken of x clamped to that range, so that a zero
+// gives itself), the IEEE sequence for small nonzero, negative and infinite
+// inputs and NaNs, behind a real branch.  Zeros stay on the fast path: a second
+// moment that never saw a nonzero gradient (zero rows of an embedding) is 0 for
+// whole waves.  Two placements of that branch, the same bits: sqrt_f32 takes one
+// side, sqrt_f32_early computes ahead of it and replaces the result.  Ahead is
+// faster where instruction issue is the bound (Dana-Star step, bfloat16 states,
+// 1.34 G elements: 10.60 against 10.73 ms), one side where memory is (ADana,
+// 51 M elements: 238.2 against 238.9 us).
+__device__ __forceinline__ bool sqrt_rare(float x, float c) { return __builtin_expect(c != x && x != 0.0f, 0); }
 __device__ __forceinline__ float sqrt_f32(float x) {
-    float s = sqrt_normal(x);
-    if (__builtin_expect(!(x >= 0x1p-96f || x == 0.0f), 0)) s = __builtin_sqrtf(opaque(x));
+    const float c = __builtin_amdgcn_fmed3f(x, 0x1p-96f, 0x1.fffffep127f);
+    if (sqrt_rare(x, c)) return __builtin_sqrtf(opaque(x));
+    return sqrt_scaled(x, __builtin_amdgcn_rsqf(c));
+}
+__device__ __forceinline__ float sqrt_f32_early(float x) {
+    const float c = __builtin_amdgcn_fmed3f(x, 0x1p-96f, 0x1.fffffep127f);
+    float s = sqrt_scaled(x, __builtin_amdgcn_rsqf(c));
+    if (sqrt_rare(x, c)) s = __builtin_sqrtf(opaque(x));
     return s;
 }
 

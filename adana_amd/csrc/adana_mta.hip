@@ -98,8 +98,11 @@ struct ScalarPack {
 // Element math
 // ---------------------------------------------------------------------------
 
-__device__ __forceinline__ float sign_f(float x) {  // torch.sign: 0 for +-0, NaN
-    return x > 0.0f ? 1.0f : (x < 0.0f ? -1.0f : 0.0f);
+// torch.sign: +0 for +-0.  A NaN gives +-1 here where torch gives 0: what it is
+// multiplied with is a NaN then too.
+__device__ __forceinline__ float sign_f(float x) {
+    const float one = __builtin_copysignf(1.0f, x);
+    return x != 0.0f ? one : 0.0f;
 }
 // torch.clamp(x, max=c), torch.clamp(x, min=c), torch.relu: NaN propagates.
 // gfx950's IEEE 754-2019 minimum / maximum (v_minimum3_f32, v_maximum3_f32),
@@ -242,9 +245,9 @@ __device__ __forceinline__ float diag_val(float x) { return NUM == NUM_FOREACH16
 
 __device__ __forceinline__ void accumulate(float (&acc)[4], float af, float g, float mfac, float m) {
     acc[0] += af;
-    acc[1] += g * g;
+    acc[1] = __builtin_fmaf(g, g, acc[1]);   // the diagnostics' own sums: one rounding each
     acc[2] += mfac;
-    acc[3] += m * m;
+    acc[3] = __builtin_fmaf(m, m, acc[3]);
 }
 
 // The end of the foreach path's update (src/optim/adana.py:345-368,
@@ -299,7 +302,7 @@ __device__ __forceinline__ StarMid star_phase_a(float g, float m, float v, float
     StarMid o;
     o.m = lerp_op<NUM>(m, g, sc);                                // :137
     o.v = ema2_op<NUM>(v, g, sc);                                // :140
-    const float sv = adana::sqrt_f32(o.v);
+    const float sv = adana::sqrt_f32_early(o.v);
     o.se = sv + sc.eps;                                          // :143
     const float ag = fabsf(g);                                   // :147
     float tu;
@@ -328,7 +331,7 @@ template <int NUM>
 __device__ __forceinline__ float star_phase_b(float p, float g, const StarMid &a, float pw,
                                               const adana_step_scalars &sc, float (&acc)[4]) {
     // tau_reg >= 1/(1+t) >= 2^-24 (t < 2^24): far above sqrt's scaling range
-    const float nt = adana::sqrt_normal(a.tr) / a.se;                   // :163-164
+    const float nt = adana::sqrt_finite(a.tr) / a.se;                   // :163-164
     const float mnt = fabsf(a.m) * nt;                           // :165
     float mfac;
     if constexpr (is_foreach(NUM)) mfac = nt * (fabsf(a.m) / a.tr);     // :474-476

@@ -5,18 +5,22 @@
 // tensor effective_time = clamp(tau * step, min=1) (src/optim/dana_star_mk4.py
 // :159, :170/:174).  The exponent is the binary32 rounding of 1 - kappa.
 //
-// Method (table-driven argument reduction, all arithmetic in binary64):
+// Method (table-driven argument reduction in base 2, all arithmetic in binary64):
 //   x = 2^e * m, m in [1, 2);  j = top 7 bits of m's fraction
 //   r = m * invc[j] - 1 (exact: invc has 12 significant bits), |r| < 0.0043
-//   (invc[j] and -ln invc[j] sit side by side: one 16-byte table load)
-//   ln x = e*ln2 + (-ln invc[j]) + log1p(r),  log1p by its degree-7 series
-//   t = y * ln x;  k = rint(t * 128 / ln2);  r' = t - k * ln2/128 (|r'| < 0.0028)
-//   x^y = 2^(k >> 7) * 2^((k & 127) / 128) * (1 + expm1(r')), degree-5 series
+//   (invc[j] and -log2 invc[j] sit side by side: one 16-byte table load)
+//   s = log2 m = -log2 invc[j] + log2(1 + r), log2(1 + r) by its degree-7 series
+//   z = 128 y log2 x = 128 y e + 128 y s;  k = rint(z);  f = z - k (exact)
+//   x^y = 2^(k >> 7) * 2^((k & 127) / 128) * 2^(f / 128), degree-5 series
 // Series truncation is below 2^-60; table entries are correctly rounded
-// binary64 values (gen_pow_tables.py).  The binary64 result is within about
-// (|t| + 4) binary64 ulps of x^y, so its binary32 rounding is the correctly
-// rounded binary32 x^y unless the result lies next to a binary32 rounding
-// boundary.
+// binary64 values (gen_pow_tables.py).  In base 2 the exponent needs no product
+// with a split ln 2 and k is taken off without one: 17 binary64 operations
+// besides the conversions, against 21 in base e.  e enters last, scaled by y, so
+// that s keeps its small absolute error.  The binary64 result is within about
+// (|t| + 4) binary64 ulps of x^y, t = y ln x (measured for 1 <= x < 2^24: at most
+// 6.7 x 2^-52; base e: 23.3), so its binary32 rounding is the
+// correctly rounded binary32 x^y unless the result lies next to a binary32
+// rounding boundary.
 //
 // Two entry points: pow_f32_unit_exp (0 < y < 1, the kernel's hot path; see
 // there why it needs no slow path) and pow_f32_via_f64 (any y: results next
@@ -65,7 +69,7 @@ __device__ __forceinline__ double fma_uc(double a, double b, double c) {
 inline double fma_uc(double a, double b, double c) { return std::fma(a, b, c); }
 #endif
 
-// binary64 x ** y for 1 <= x < 3e38 (finite).  Writes t = y * ln x.  The
+// binary64 x ** y for 1 <= x < 3e38 (finite).  Writes t = y * ln x (nearly).  The
 // tables are passed in so that a kernel can read them from a copy in LDS (the
 // per-lane gathers then stay off the vector-memory path that the streaming
 // loads use); pow_core_f64 reads the global tables.
@@ -77,32 +81,31 @@ ADANA_HD inline double pow_core_tab(float x, float y, double &t_out, const LogPa
     const double m = static_cast<double>(bits_as<float>((xb & 0x007fffffu) | 0x3f800000u));
     const LogPair c = log_tab[j];
     const double r = std::fma(m, c.inv_c, -1.0);
-    // log1p(r) = r + r^2 * (-1/2 + r/3 - r^2/4 + r^3/5 - r^4/6 + r^5/7)
-    double q = 1.0 / 7.0;
-    q = fma_uc(q, r, -1.0 / 6.0);
-    q = fma_uc(q, r, 1.0 / 5.0);
-    q = fma_uc(q, r, -1.0 / 4.0);
-    q = fma_uc(q, r, 1.0 / 3.0);
-    q = fma_uc(q, r, -0.5);
-    const double lp = std::fma(r * r, q, r);
-    // ln 2 split so that e * LN2_HI and k * LN2_HI / 128 are exact
-    const double LN2_HI = 6.93147180369123816490e-01;
-    const double LN2_LO = 1.90821492927058770002e-10;
-    const double ed = static_cast<double>(e);
-    const double lnx = std::fma(ed, LN2_HI, c.neg_log) + std::fma(ed, LN2_LO, lp);
-    const double t = static_cast<double>(y) * lnx;
-    // e^t = 2^(k/128) e^r'
-    const double kd = std::rint(t * 184.66496523378731);        // 128 / ln 2
-    double rr = std::fma(-kd, LN2_HI / 128.0, t);
-    rr = std::fma(-kd, LN2_LO / 128.0, rr);
-    double p = 1.0 / 120.0;
-    p = fma_uc(p, rr, 1.0 / 24.0);
-    p = fma_uc(p, rr, 1.0 / 6.0);
-    p = fma_uc(p, rr, 0.5);
-    p = std::fma(rr * rr, p, rr);                                // expm1(r')
+    // log2(1 + r) = r * (c1 + r * (-c1/2 + r * (c1/3 ...))), c1 = 1 / ln 2
+    const double c1 = 1.4426950408889634;
+    double q = c1 / 7.0;
+    q = fma_uc(q, r, c1 / -6.0);
+    q = fma_uc(q, r, c1 / 5.0);
+    q = fma_uc(q, r, c1 / -4.0);
+    q = fma_uc(q, r, c1 / 3.0);
+    q = fma_uc(q, r, c1 / -2.0);
+    q = fma_uc(q, r, c1);
+    const double s = std::fma(r, q, c.neg_log2);
+    const double y128 = static_cast<double>(y) * 128.0;           // exact
+    const double z = std::fma(static_cast<double>(e), y128, s * y128);
+    // 2^(z / 128) = 2^(k / 128) 2^(f / 128); d_i = (ln 2 / 128)^i / i!
+    const double kd = std::rint(z);
+    const double f = z - kd;
+    const double ln2_128 = 6.93147180559945286e-01 / 128.0;
+    double p = ln2_128 * ln2_128 * ln2_128 * ln2_128 * ln2_128 / 120.0;
+    p = fma_uc(p, f, ln2_128 * ln2_128 * ln2_128 * ln2_128 / 24.0);
+    p = fma_uc(p, f, ln2_128 * ln2_128 * ln2_128 / 6.0);
+    p = fma_uc(p, f, ln2_128 * ln2_128 / 2.0);
+    p = fma_uc(p, f, ln2_128);
+    p *= f;                                                       // 2^(f / 128) - 1
     const int k = static_cast<int>(kd);
     const double tj = exp_tab[k & 127];
-    t_out = t;
+    t_out = z * ln2_128;
     return std::ldexp(std::fma(tj, p, tj), k >> 7);
 }
 

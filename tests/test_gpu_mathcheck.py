@@ -80,3 +80,10 @@ def test_sqrt_f32_exhaustive():
     print("case: sqrt_f32 exhaustive", flush=True)
     bad, first = _run(5, 0, 0xFFFFFFFF)
     assert bad == 0, f"{bad} mismatches, first pattern {first:#010x}"
+
+
+def test_sqrt_f32_early_exhaustive():
+    """sqrt_f32_early(x) == sqrtf(x) bit for bit on all 2^32 binary32 patterns."""
+    print("case: sqrt_f32_early exhaustive", flush=True)
+    bad, first = _run(6, 0, 0xFFFFFFFF)
+    assert bad == 0, f"{bad} mismatches, first pattern {first:#010x}"
