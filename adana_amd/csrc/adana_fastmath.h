@@ -49,6 +49,19 @@ __device__ __forceinline__ float div_core(float a, float b) {
     return __builtin_fmaf(r, y, q);
 }
 
+// Correctly rounded a / b for b in [2^-66, 2^21] and a +0 or in [2^-98, 2^86],
+// a / b below 2^110: the reciprocal with one Newton step, the quotient and one
+// remainder correction.  Nothing under- or overflows there, so only the mantissas
+// matter; checked for all 2^46 pairs of them (without the Newton step 47,045 pairs
+// round the wrong way).  6 instructions against the IEEE sequence's 11.
+__device__ __forceinline__ float div_short(float a, float b) {
+    float y = __builtin_amdgcn_rcpf(b);
+    y = __builtin_fmaf(__builtin_fmaf(-b, y, 1.0f), y, y);
+    const float q = a * y;
+    const float r = __builtin_fmaf(-b, q, a);
+    return __builtin_fmaf(r, y, q);
+}
+
 // Correctly rounded sqrt for finite x >= 2^-96: x * rsqrt(x) by the hardware
 // reciprocal square root and one remainder correction (checked for every such
 // binary32 x).  5 instructions; the hardware square root with a test of both
@@ -72,7 +85,7 @@ __device__ __forceinline__ float sqrt_normal(float x) { return x < __builtin_inf
 // whole waves.  Two placements of that branch, the same bits: sqrt_f32 takes one
 // side, sqrt_f32_early computes ahead of it and replaces the result.  Ahead is
 // faster where instruction issue is the bound (Dana-Star step, bfloat16 states,
-// 1.34 G elements: 10.60 against 10.73 ms), one side where memory is (ADana,
+// 2.7 G elements: 10.60 against 10.73 ms), one side where memory is (ADana,
 // 51 M elements: 238.2 against 238.9 us).
 __device__ __forceinline__ bool sqrt_rare(float x, float c) { return __builtin_expect(c != x && x != 0.0f, 0); }
 __device__ __forceinline__ float sqrt_f32(float x) {

@@ -14,6 +14,8 @@
 //              bfloat16 patterns [lo, hi] (hi <= 0xffff)
 //   which = 5: sqrt_f32(x) vs sqrtf(x) for the binary32 patterns [lo, hi]
 //   which = 6: sqrt_f32_early(x) vs sqrtf(x) for the binary32 patterns [lo, hi]
+//   which = 7: div_short(a, b) vs a / b: b's mantissa is the pattern's low 23 bits,
+//              a's and both exponents a hash of the pattern
 // out[0] counts mismatching patterns, out[1] holds the smallest one.
 #include <hip/hip_runtime.h>
 
@@ -59,6 +61,18 @@ __global__ void check_kernel(int which, uint32_t lo, uint64_t count, unsigned lo
             const float v = __uint_as_float(bits << 16);
             got = adana::bf16_round(adana::sqrt_bf16(v));
             ref = adana::bf16_round(sqrtf(v));
+        } else if (which == 7) {
+            uint64_t h = (bits + 1ull) * 0x9E3779B97F4A7C15ull;
+            h = (h ^ (h >> 29)) * 0xBF58476D1CE4E5B9ull;
+            h ^= h >> 32;
+            const int eb = static_cast<int>((h >> 23) % 87) - 66;                   // [-66, 20]
+            int ea = static_cast<int>((h >> 40) % 184) - 98;                        // [-98, 85]
+            if (ea > eb + 109) ea = eb + 109;
+            const float b = ldexpf(__uint_as_float((bits & 0x7fffffu) | 0x3f800000u), eb);
+            float a = ldexpf(__uint_as_float((static_cast<uint32_t>(h) & 0x7fffffu) | 0x3f800000u), ea);
+            if ((h >> 56) == 0) a = 0.0f;
+            got = adana::div_short(a, b);
+            ref = a / b;
         } else {
             got = which == 5 ? adana::sqrt_f32(x) : adana::sqrt_f32_early(x);
             ref = sqrtf(x);
@@ -74,7 +88,7 @@ __global__ void check_kernel(int which, uint32_t lo, uint64_t count, unsigned lo
 
 extern "C" int adana_mathcheck(int which, uint32_t lo, uint32_t hi, unsigned long long *d_out,
                                void *stream) {
-    if (hi < lo || which < 0 || which > 6 || (which == 4 && hi > 0xffffu) || !d_out) return -1;
+    if (hi < lo || which < 0 || which > 7 || (which == 4 && hi > 0xffffu) || !d_out) return -1;
     const uint64_t count = static_cast<uint64_t>(hi) - lo + 1;
     hipLaunchKernelGGL(check_kernel, dim3(8192), dim3(256), 0, static_cast<hipStream_t>(stream), which, lo,
                        count, d_out);
