@@ -860,53 +860,53 @@ __global__ __launch_bounds__(kSmallThreads) void segment_few_kernel(Args a) {
     const int tid = threadIdx.x;
     const uint32_t n = a.n_few[0];
     for (uint32_t slot = blockIdx.x; slot < n; slot += gridDim.x) {
-    const Segment s = a.seg[a.few[slot]];
-    __syncthreads();                                 // s_lo and the others are read by the segment before
-    const uint32_t *p = a.cand + s.first;
-    if (tid == 0) {
-        s_lo = 0xffffffffu;
-        s_hi = 0;
-        s_less[0] = s_less[1] = 0;
-    }
-    uint32_t key[kSmallPer];
-    uint32_t mn = 0xffffffffu, mx = 0, l0 = 0, l1 = 0;
-#pragma unroll
-    for (int u = 0; u < kSmallPer; ++u) {
-        const uint32_t i = tid + u * kSmallThreads;
-        key[u] = i < s.count ? p[i] : 0u;
-    }
-#pragma unroll
-    for (int u = 0; u < kSmallPer; ++u) {
-        if (tid + u * kSmallThreads < s.count) {
-            mn = min(mn, key[u]);
-            mx = max(mx, key[u]);
-            l0 += s.n_heavy > 0 && key[u] < s.heavy_key[0];
-            l1 += s.n_heavy > 1 && key[u] < s.heavy_key[1];
+        const Segment s = a.seg[a.few[slot]];
+        __syncthreads();                                 // s_lo and the others are read by the segment before
+        const uint32_t *p = a.cand + s.first;
+        if (tid == 0) {
+            s_lo = 0xffffffffu;
+            s_hi = 0;
+            s_less[0] = s_less[1] = 0;
         }
-    }
-    mn = wave_min(mn);
-    mx = wave_max(mx);
-    __syncthreads();
-    if ((tid & 63) == 0) {
-        atomicMin(&s_lo, mn);
-        atomicMax(&s_hi, mx);
-    }
-    if (s.n_heavy) {
-        if (l0) atomicAdd(&s_less[0], l0);
-        if (l1) atomicAdd(&s_less[1], l1);
-    }
-    __syncthreads();
-    const uint32_t lo = s_lo, hi = s_hi, less[kHeavy] = {s_less[0], s_less[1]};
-    for (uint32_t j = 0; j < s.n_ranks; ++j) {
-        uint32_t r = a.residual[s.rank_first + j], k = lo;
-        if (!on_heavy(s, less, r, k) && s.count)
-            k = select_rank<kSmallThreads>(r, lo, hi, h, waves, s_digit, [&](auto f) {
+        uint32_t key[kSmallPer];
+        uint32_t mn = 0xffffffffu, mx = 0, l0 = 0, l1 = 0;
 #pragma unroll
-                for (int u = 0; u < kSmallPer; ++u)
-                    if (tid + u * kSmallThreads < s.count) f(key[u]);
-            });
-        if (tid == 0) a.out[s.rank_first + j] = key_bits(k);
-    }
+        for (int u = 0; u < kSmallPer; ++u) {
+            const uint32_t i = tid + u * kSmallThreads;
+            key[u] = i < s.count ? p[i] : 0u;
+        }
+#pragma unroll
+        for (int u = 0; u < kSmallPer; ++u) {
+            if (tid + u * kSmallThreads < s.count) {
+                mn = min(mn, key[u]);
+                mx = max(mx, key[u]);
+                l0 += s.n_heavy > 0 && key[u] < s.heavy_key[0];
+                l1 += s.n_heavy > 1 && key[u] < s.heavy_key[1];
+            }
+        }
+        mn = wave_min(mn);
+        mx = wave_max(mx);
+        __syncthreads();
+        if ((tid & 63) == 0) {
+            atomicMin(&s_lo, mn);
+            atomicMax(&s_hi, mx);
+        }
+        if (s.n_heavy) {
+            if (l0) atomicAdd(&s_less[0], l0);
+            if (l1) atomicAdd(&s_less[1], l1);
+        }
+        __syncthreads();
+        const uint32_t lo = s_lo, hi = s_hi, less[kHeavy] = {s_less[0], s_less[1]};
+        for (uint32_t j = 0; j < s.n_ranks; ++j) {
+            uint32_t r = a.residual[s.rank_first + j], k = lo;
+            if (!on_heavy(s, less, r, k) && s.count)
+                k = select_rank<kSmallThreads>(r, lo, hi, h, waves, s_digit, [&](auto f) {
+#pragma unroll
+                    for (int u = 0; u < kSmallPer; ++u)
+                        if (tid + u * kSmallThreads < s.count) f(key[u]);
+                });
+            if (tid == 0) a.out[s.rank_first + j] = key_bits(k);
+        }
     }
 }
 
@@ -931,171 +931,171 @@ __global__ __launch_bounds__(kSegThreads) void segment_many_kernel(Args a) {
     const int tid = threadIdx.x;
     const uint32_t n = a.n_few[1];
     for (uint32_t slot = blockIdx.x; slot < n; slot += gridDim.x) {
-    const Segment s = a.seg[a.many[slot]];
-    __syncthreads();                                 // LDS is read by the segment before
-    const uint32_t *p = a.cand + s.first;
-    if (tid == 0) {
-        s_lo = 0xffffffffu;
-        s_hi = 0;
-        s_less[0] = s_less[1] = 0;
-        s_fail = 0;
-    }
-    __syncthreads();
-    uint32_t mn = 0xffffffffu, mx = 0, l0 = 0, l1 = 0;
-    each_key<kSegThreads>(p, s.count, [&](uint32_t, uint32_t k) {
-        mn = min(mn, k);
-        mx = max(mx, k);
-        l0 += s.n_heavy > 0 && k < s.heavy_key[0];
-        l1 += s.n_heavy > 1 && k < s.heavy_key[1];
-    });
-    mn = wave_min(mn);
-    mx = wave_max(mx);
-    if ((tid & 63) == 0) {
-        atomicMin(&s_lo, mn);
-        atomicMax(&s_hi, mx);
-    }
-    if (s.n_heavy) {
-        if (l0) atomicAdd(&s_less[0], l0);
-        if (l1) atomicAdd(&s_less[1], l1);
-    }
-    __syncthreads();
-    const uint32_t lo = s_lo, hi = s_hi, less[kHeavy] = {s_less[0], s_less[1]};
-    if (s.n_ranks <= 4) {
-        for (uint32_t j = 0; j < s.n_ranks; ++j) {
-            uint32_t r = a.residual[s.rank_first + j], k = lo;
-            if (!on_heavy(s, less, r, k) && s.count)
-                k = select_rank<kSegThreads>(r, lo, hi, h, waves, s_digit, [&](auto f) {
-                    each_key<kSegThreads>(p, s.count, [&](uint32_t, uint32_t key) { f(key); });
-                });
-            if (tid == 0) a.out[s.rank_first + j] = key_bits(k);
+        const Segment s = a.seg[a.many[slot]];
+        __syncthreads();                                 // LDS is read by the segment before
+        const uint32_t *p = a.cand + s.first;
+        if (tid == 0) {
+            s_lo = 0xffffffffu;
+            s_hi = 0;
+            s_less[0] = s_less[1] = 0;
+            s_fail = 0;
         }
-        continue;
-    }
-    for (uint32_t j = tid; j < s.n_ranks; j += kSegThreads) {
-        uint32_t r = a.residual[s.rank_first + j], k;
-        const bool rep = on_heavy(s, less, r, k);
-        if (rep) {
-            // (its place: the candidates below it, so that places stay in order)
-            r = s.n_heavy > 1 && k == s.heavy_key[1] ? less[1] : less[0];
-            a.out[s.rank_first + j] = key_bits(k);
-        }
-        place[j] = 2 * r + (rep ? 1u : 0u);
-    }
-    if (s.count == 0) continue;
-    if (s.count <= static_cast<uint32_t>(kSegSort)) {
-        const int pw = pow2_at_least(s.count);
-        for (uint32_t i = tid; i < static_cast<uint32_t>(pw); i += kSegThreads) x[i] = i < s.count ? p[i] : 0xffffffffu;
-        lds_sort<kSegThreads>(x, pw);                // (its first step waits for place too)
-        for (uint32_t j = tid; j < s.n_ranks; j += kSegThreads)
-            if (!(place[j] & 1u)) a.out[s.rank_first + j] = key_bits(x[min(place[j] >> 1, s.count - 1)]);
-        continue;
-    }
-    if (tid == 0) {
-        r_from[0] = lo;
-        r_width[0] = hi - lo;
-        r_base[0] = 0;
-        n_range = 1;
-    }
-    __syncthreads();
-    // first rank (index into place) at or past candidate place c
-    auto first_at = [&](uint32_t c) {
-        uint32_t l = 0, u = s.n_ranks;
-        while (l < u) {
-            const uint32_t mid = (l + u) >> 1;
-            if ((place[mid] >> 1) < c) l = mid + 1; else u = mid;
-        }
-        return l;
-    };
-    while (true) {
-        const uint32_t left = n_range;
         __syncthreads();
-        if (left == 0 || s_fail) break;              // uniform
-        const uint32_t from = r_from[left - 1], width = r_width[left - 1], base = r_base[left - 1];
-        for (int i = tid; i < kParts; i += kSegThreads) h[i] = 0;
-        __syncthreads();
-        if (tid == 0) n_range = left - 1;
-        const int sh = part_shift(width, kPartBits);
+        uint32_t mn = 0xffffffffu, mx = 0, l0 = 0, l1 = 0;
         each_key<kSegThreads>(p, s.count, [&](uint32_t, uint32_t k) {
-            const uint32_t d = k - from;
-            if (d <= width) atomicAdd(&h[d >> sh], 1u);
+            mn = min(mn, k);
+            mx = max(mx, k);
+            l0 += s.n_heavy > 0 && k < s.heavy_key[0];
+            l1 += s.n_heavy > 1 && k < s.heavy_key[1];
         });
+        mn = wave_min(mn);
+        mx = wave_max(mx);
+        if ((tid & 63) == 0) {
+            atomicMin(&s_lo, mn);
+            atomicMax(&s_hi, mx);
+        }
+        if (s.n_heavy) {
+            if (l0) atomicAdd(&s_less[0], l0);
+            if (l1) atomicAdd(&s_less[1], l1);
+        }
         __syncthreads();
-        constexpr int kPerT = kParts / kSegThreads;
-        uint32_t c[kPerT], sum = 0, all;
-#pragma unroll
-        for (int k = 0; k < kPerT; ++k) sum += c[k] = h[tid * kPerT + k];
-        const uint32_t start = base + block_scan<kSegThreads>(sum, waves, &all);
-        bool sorted[kPerT];
-        uint32_t before = start, want = 0;
-#pragma unroll
-        for (int k = 0; k < kPerT; ++k) {
-            const uint32_t j0 = first_at(before), j1 = first_at(before + c[k]);
-            sorted[k] = j1 > j0;
-            if (j1 > j0 && (sh == 0 || c[k] > kGroup)) {
-                // one key, or a range of its own
-                sorted[k] = false;
-                const uint32_t key = from + (static_cast<uint32_t>(tid * kPerT + k) << sh);
-                if (sh == 0) {
-                    for (uint32_t j = j0; j < j1; ++j)
-                        if (!(place[j] & 1u)) a.out[s.rank_first + j] = key_bits(key);
-                } else {
-                    const uint32_t at = atomicAdd(&n_range, 1u);
-                    if (at < kRanges) {
-                        r_from[at] = key;
-                        r_width[at] = min((1u << sh) - 1u, from + width - key);
-                        r_base[at] = before;
-                    } else {
-                        s_fail = 1;
-                    }
-                }
+        const uint32_t lo = s_lo, hi = s_hi, less[kHeavy] = {s_less[0], s_less[1]};
+        if (s.n_ranks <= 4) {
+            for (uint32_t j = 0; j < s.n_ranks; ++j) {
+                uint32_t r = a.residual[s.rank_first + j], k = lo;
+                if (!on_heavy(s, less, r, k) && s.count)
+                    k = select_rank<kSegThreads>(r, lo, hi, h, waves, s_digit, [&](auto f) {
+                        each_key<kSegThreads>(p, s.count, [&](uint32_t, uint32_t key) { f(key); });
+                    });
+                if (tid == 0) a.out[s.rank_first + j] = key_bits(k);
             }
-            want += sorted[k] ? c[k] : 0u;
-            before += c[k];
+            continue;
         }
-        uint32_t total;
-        uint32_t at = block_scan<kSegThreads>(want, waves, &total);
-        // h: a part's group (wanted candidates before it / kGroup)
-#pragma unroll
-        for (int k = 0; k < kPerT; ++k) {
-            h[tid * kPerT + k] = sorted[k] ? at / kGroup : kNot;
-            at += sorted[k] ? c[k] : 0u;
+        for (uint32_t j = tid; j < s.n_ranks; j += kSegThreads) {
+            uint32_t r = a.residual[s.rank_first + j], k;
+            const bool rep = on_heavy(s, less, r, k);
+            if (rep) {
+                // (its place: the candidates below it, so that places stay in order)
+                r = s.n_heavy > 1 && k == s.heavy_key[1] ? less[1] : less[0];
+                a.out[s.rank_first + j] = key_bits(k);
+            }
+            place[j] = 2 * r + (rep ? 1u : 0u);
         }
-        at -= want;
-        for (uint32_t g = 0; g * kGroup < total; ++g) {
-            if (tid == 0) s_n = 0;
+        if (s.count == 0) continue;
+        if (s.count <= static_cast<uint32_t>(kSegSort)) {
+            const int pw = pow2_at_least(s.count);
+            for (uint32_t i = tid; i < static_cast<uint32_t>(pw); i += kSegThreads) x[i] = i < s.count ? p[i] : 0xffffffffu;
+            lds_sort<kSegThreads>(x, pw);                // (its first step waits for place too)
+            for (uint32_t j = tid; j < s.n_ranks; j += kSegThreads)
+                if (!(place[j] & 1u)) a.out[s.rank_first + j] = key_bits(x[min(place[j] >> 1, s.count - 1)]);
+            continue;
+        }
+        if (tid == 0) {
+            r_from[0] = lo;
+            r_width[0] = hi - lo;
+            r_base[0] = 0;
+            n_range = 1;
+        }
+        __syncthreads();
+        // first rank (index into place) at or past candidate place c
+        auto first_at = [&](uint32_t c) {
+            uint32_t l = 0, u = s.n_ranks;
+            while (l < u) {
+                const uint32_t mid = (l + u) >> 1;
+                if ((place[mid] >> 1) < c) l = mid + 1; else u = mid;
+            }
+            return l;
+        };
+        while (true) {
+            const uint32_t left = n_range;
             __syncthreads();
+            if (left == 0 || s_fail) break;              // uniform
+            const uint32_t from = r_from[left - 1], width = r_width[left - 1], base = r_base[left - 1];
+            for (int i = tid; i < kParts; i += kSegThreads) h[i] = 0;
+            __syncthreads();
+            if (tid == 0) n_range = left - 1;
+            const int sh = part_shift(width, kPartBits);
             each_key<kSegThreads>(p, s.count, [&](uint32_t, uint32_t k) {
                 const uint32_t d = k - from;
-                if (d <= width && h[d >> sh] == g) {
-                    const uint32_t e = atomicAdd(&s_n, 1u);
-                    if (e < static_cast<uint32_t>(kSegSort)) x[e] = k;
-                }
+                if (d <= width) atomicAdd(&h[d >> sh], 1u);
             });
             __syncthreads();
-            const uint32_t m = min(s_n, static_cast<uint32_t>(kSegSort));
-            const int pw = pow2_at_least(m);
-            for (uint32_t i = m + tid; i < static_cast<uint32_t>(pw); i += kSegThreads) x[i] = 0xffffffffu;
-            lds_sort<kSegThreads>(x, pw);
-            // each part's first candidate in the sorted group is where its keys begin
-            uint32_t b = start;
+            constexpr int kPerT = kParts / kSegThreads;
+            uint32_t c[kPerT], sum = 0, all;
+#pragma unroll
+            for (int k = 0; k < kPerT; ++k) sum += c[k] = h[tid * kPerT + k];
+            const uint32_t start = base + block_scan<kSegThreads>(sum, waves, &all);
+            bool sorted[kPerT];
+            uint32_t before = start, want = 0;
 #pragma unroll
             for (int k = 0; k < kPerT; ++k) {
-                if (sorted[k] && h[tid * kPerT + k] == g && m) {
+                const uint32_t j0 = first_at(before), j1 = first_at(before + c[k]);
+                sorted[k] = j1 > j0;
+                if (j1 > j0 && (sh == 0 || c[k] > kGroup)) {
+                    // one key, or a range of its own
+                    sorted[k] = false;
                     const uint32_t key = from + (static_cast<uint32_t>(tid * kPerT + k) << sh);
-                    uint32_t l = 0, u = m;
-                    while (l < u) {
-                        const uint32_t mid = (l + u) >> 1;
-                        if (x[mid] < key) l = mid + 1; else u = mid;
+                    if (sh == 0) {
+                        for (uint32_t j = j0; j < j1; ++j)
+                            if (!(place[j] & 1u)) a.out[s.rank_first + j] = key_bits(key);
+                    } else {
+                        const uint32_t at = atomicAdd(&n_range, 1u);
+                        if (at < kRanges) {
+                            r_from[at] = key;
+                            r_width[at] = min((1u << sh) - 1u, from + width - key);
+                            r_base[at] = before;
+                        } else {
+                            s_fail = 1;
+                        }
                     }
-                    for (uint32_t j = first_at(b); j < s.n_ranks && (place[j] >> 1) < b + c[k]; ++j)
-                        if (!(place[j] & 1u)) a.out[s.rank_first + j] = key_bits(x[min(l + (place[j] >> 1) - b, m - 1)]);
                 }
-                b += c[k];
+                want += sorted[k] ? c[k] : 0u;
+                before += c[k];
             }
-            __syncthreads();
+            uint32_t total;
+            uint32_t at = block_scan<kSegThreads>(want, waves, &total);
+            // h: a part's group (wanted candidates before it / kGroup)
+#pragma unroll
+            for (int k = 0; k < kPerT; ++k) {
+                h[tid * kPerT + k] = sorted[k] ? at / kGroup : kNot;
+                at += sorted[k] ? c[k] : 0u;
+            }
+            at -= want;
+            for (uint32_t g = 0; g * kGroup < total; ++g) {
+                if (tid == 0) s_n = 0;
+                __syncthreads();
+                each_key<kSegThreads>(p, s.count, [&](uint32_t, uint32_t k) {
+                    const uint32_t d = k - from;
+                    if (d <= width && h[d >> sh] == g) {
+                        const uint32_t e = atomicAdd(&s_n, 1u);
+                        if (e < static_cast<uint32_t>(kSegSort)) x[e] = k;
+                    }
+                });
+                __syncthreads();
+                const uint32_t m = min(s_n, static_cast<uint32_t>(kSegSort));
+                const int pw = pow2_at_least(m);
+                for (uint32_t i = m + tid; i < static_cast<uint32_t>(pw); i += kSegThreads) x[i] = 0xffffffffu;
+                lds_sort<kSegThreads>(x, pw);
+                // each part's first candidate in the sorted group is where its keys begin
+                uint32_t b = start;
+#pragma unroll
+                for (int k = 0; k < kPerT; ++k) {
+                    if (sorted[k] && h[tid * kPerT + k] == g && m) {
+                        const uint32_t key = from + (static_cast<uint32_t>(tid * kPerT + k) << sh);
+                        uint32_t l = 0, u = m;
+                        while (l < u) {
+                            const uint32_t mid = (l + u) >> 1;
+                            if (x[mid] < key) l = mid + 1; else u = mid;
+                        }
+                        for (uint32_t j = first_at(b); j < s.n_ranks && (place[j] >> 1) < b + c[k]; ++j)
+                            if (!(place[j] & 1u)) a.out[s.rank_first + j] = key_bits(x[min(l + (place[j] >> 1) - b, m - 1)]);
+                    }
+                    b += c[k];
+                }
+                __syncthreads();
+            }
         }
-    }
-    if (s_fail && tid == 0) a.state[s.tensor] = kRadix;
+        if (s_fail && tid == 0) a.state[s.tensor] = kRadix;
     }
 }
 

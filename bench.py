@@ -755,8 +755,8 @@ def consumer_bench(args):
     ms = (time.perf_counter() - t0) * 1e3 / args.steps
     select_ms = None
     if plain is not None:
-        # the device selection alone (no result dictionaries), with and without
-        # compaction, interleaved call by call
+        # the device selection alone (no result dictionaries), the two-read form
+        # (compact) and the radix select, interleaved call by call
         t = {True: [], False: []}
         for rep in range(args.steps + 1):
             for c in (True, False):
@@ -768,8 +768,9 @@ def consumer_bench(args):
                     t[c].append((time.perf_counter() - t0) * 1e3)
         select_ms = {"compaction": round(float(np.median(t[True])), 4),
                      "no_compaction": round(float(np.median(t[False])), 4),
-                     "note": "median over the steps of the device selection alone (adana_order_stats), "
-                             "interleaved; compaction is the default"}
+                     "note": "median over the steps of the device selection alone, interleaved: "
+                             "compaction (the default) is adana_order_stats_sampled, no_compaction "
+                             "adana_order_stats"}
     # the reference's host path, timed on a bounded sample
     if tau:
         sample = [t for t in taus][:4]                            # first four tensors of the list
