@@ -88,7 +88,7 @@ def workload(name):
                     grad_note="N(0,1e-3); embedding rows nonzero w.p. 0.1")
     if name == "north_star_clip":
         w = workload("north_star")
-        w.update(name=name, clip=0.5, grad_note=w["grad_note"] + "; clip_grad_norm_(0.5) each step")
+        w.update(name=name, clip=0.5, grad_note=w["grad_note"] + "; clip_grad_norm_(0.5 * 0.99^k) at step k")
         return w
     if name == "north_star_bf16":
         # the reference's own bfloat16 path: bfloat16 parameters and gradients make m, v, tau
@@ -994,7 +994,9 @@ def main():
 
     def one_step(_k):
         if w.get("clip"):
-            grad_norms.append(opt.clip_grad_norm_(w["clip"]).item())   # src/optim/base.py:250-257
+            # src/optim/base.py:250-257; the bound falls by 1% a step, so that every
+            # step scales the stored gradients (at a coefficient of 1 it would not)
+            grad_norms.append(opt.clip_grad_norm_(w["clip"] * 0.99 ** len(grad_norms)).item())
         opt.step()
         if sched is not None:
             sched.step()

@@ -82,3 +82,22 @@ def test_large_bins():
     (got,) = order_values([x], [ranks])
     want = torch.sort(x)[0][torch.tensor(ranks, device=DEV)].cpu().numpy()
     assert np.array_equal(got, want)
+
+
+@pytest.mark.parametrize("outliers", [0, 2000])
+@pytest.mark.parametrize("width", [1, 3, 40, 300])
+def test_clusters_of_few_keys(width, outliers):
+    """Nearly all values on ``width`` neighbouring floats, the rest spread over
+    many decades: too narrow for the bins, so left to the radix select (by the
+    sample, or after the first read): the same values as np.sort's."""
+    from adana_amd.tau_stats import order_values
+
+    print("case: cluster", width, outliers, flush=True)
+    rng = np.random.default_rng(width)
+    n = 200_000
+    x = (np.float32(0.25).view(np.int32) + rng.integers(0, width, n).astype(np.int32)).view(np.float32)
+    at = rng.choice(n, outliers, replace=False)
+    x[at] = (10.0 ** rng.uniform(-30, 0, outliers)).astype(np.float32)
+    ranks = np.unique(np.concatenate([np.arange(0, n, 997), [0, n - 1]])).astype(np.int64)
+    got = order_values([torch.from_numpy(x).to(DEV)], [ranks])[0]
+    np.testing.assert_array_equal(np.asarray(got), np.sort(x)[ranks])
